@@ -7,7 +7,7 @@
 namespace duct {
 
 constexpr int kXprodMaxM = 64;    // the dense kernels' largest complex x-mode count (2/3 rule: mx1 + 1)
-constexpr int kXprodMaxX = 192;   // and physical x point count (mgalx); rocFFT past them
+constexpr int kXprodMaxX = 192;   // and physical x point count (mgalx)
 
 struct XprodArgs {
     const d2v* in[3];      // u, v, w: complex(8) (m, m, M)
@@ -22,6 +22,31 @@ hipError_t launch_xprod(const XprodArgs& a, hipStream_t st);
 // lanes of DPP rows (xlane.hip; Einv and Fwd unused); tab = build_xlane_table on the device.
 hipError_t launch_xprod_lane(const XprodArgs& a, const d2v* tab, hipStream_t st);
 void build_xlane_table(std::vector<double>& tab);
+
+// The same products for an even X of factors 2, 3 and 5 (xprod_fft.hip; Einv and Fwd unused); tw =
+// build_xfft_table on the device: (cos, sin)(2 pi n / X), n < X.
+constexpr int xfft_per_thread(int R) { return R == 4 ? 8 : 12; }   // complex points of the lines per thread
+constexpr int kXfftMaxThreads = 512;
+constexpr int kXfftMaxX = 2048;        // two lines of a workgroup's minimum fill 512 threads
+constexpr int kXfftMaxPasses = 6;      // besides the fused radix
+struct XfftPass {
+    int r, ns, nb, tw;                 // radix, length already transformed, X / r, X / (ns r)
+    float inv_nb, inv_ns;
+};
+struct XprodFftArgs {
+    const d2v* in[3];
+    d2v* out[6];
+    const d2v* tw;
+    long lines, tiles;
+    double scale;                      // 1 / (2 X)
+    float inv_nf, inv_nz;              // 1 / (X / R), 1 / (X - 2 M + 1)
+    int M, X, T, logT, ld;             // T = 2^logT lines per workgroup, ld: stride of a line's LDS image
+    int ninv, nfwd;
+    XfftPass inv[kXfftMaxPasses], fwd[kXfftMaxPasses];
+};
+bool xprod_fft_supported(int M, int X);
+void build_xfft_table(int X, std::vector<double>& tab);
+hipError_t launch_xprod_fft(const XprodArgs& a, const d2v* tw, hipStream_t st);
 
 struct FourxArgs {
     d2v* fou;              // fou(0:M-1, lines) complex, mode fastest

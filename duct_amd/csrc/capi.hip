@@ -144,6 +144,8 @@ struct Lib {
     double* xdft[2] = {nullptr, nullptr}; // advection x-DFTs (inverse, forward), fragment layout
     d2v* xlane = nullptr;                  // twiddles of the 192-point lane FFTs (build_xlane_table)
     int xdft_M = 0, xdft_X = 0;
+    d2v* xtw = nullptr;                   // roots of unity of k_xprod_fft (build_xfft_table)
+    int xtw_X = 0;
     d2v* prods = nullptr;                 // the six product fields of the advection term
     size_t prods_bytes = 0;
     // x-transforms past the dense kernels' sizes: rocFFT plans (kept per layout), their work
@@ -1085,6 +1087,21 @@ int ensure_xdft(int M, int X)
     return OK;
 }
 
+// The roots of unity of the X-point transforms of k_xprod_fft, rebuilt when X changes.
+int ensure_xtw(int X)
+{
+    if (L.xtw_X == X) return OK;
+    std::vector<double> tab;
+    build_xfft_table(X, tab);
+    HIPCHK(hipStreamSynchronize(L.stream));
+    free_ptr(L.xtw);
+    L.xtw_X = 0;
+    HIPCHK(hipMalloc((void**)&L.xtw, tab.size() * sizeof(double)));
+    HIPCHK(hipMemcpy(L.xtw, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
+    L.xtw_X = X;
+    return OK;
+}
+
 // Independent derivative products (y or z, each its own field, matrix, scale and beta) in one
 // launch on the library's stream, with the derivative matrices of duct_setup_ (padded to L.dc_np).
 int cline_run(int mm, int M, std::initializer_list<ClineOp> ops)
@@ -1106,8 +1123,7 @@ int cline_run(int mm, int M, std::initializer_list<ClineOp> ops)
 // k_xprod, then the nine derivative terms in the order of operators.F:91-272 per output
 // (adv1: uu_x, uv_y, uw_z; adv2: vv_y, uv_x, vw_z; adv3: ww_z, uw_x, vw_y); the caller has
 // checked the sizes.
-// The dense x-DFT kernels (k_xprod, k_fourx) cover M % 16 == 0, M <= 64, X % 16 == 0, X <= 192;
-// other sizes go through batched rocFFT real transforms.
+// The dense x-DFT kernels (k_xprod, k_fourx) cover M % 16 == 0, M <= 64, X % 16 == 0, X <= 192.
 bool dense_x(int M, int X)
 {
     return M % 16 == 0 && M <= kXprodMaxM && X % 16 == 0 && X <= kXprodMaxX;
@@ -1166,7 +1182,8 @@ int xfft_run(bool forward, void* in, void* out, size_t X, size_t batch, size_t i
     return OK;
 }
 
-// The six products of the advection term (k_xprod's output, prods (m, m, M) each) through rocFFT:
+// The six products of the advection term (k_xprod's output, prods (m, m, M) each) through rocFFT,
+// for the x grids that k_xprod_fft does not take (a factor past 5, or more than kXfftMaxX points):
 // fill (modes M..X/2 zero), c2r of u, v, w, the products in physical space, r2c, pack with 1/X.
 int xprod_fft(const d2v* const in[3], d2v* prods, int mm, int M, int X)
 {
@@ -1204,7 +1221,11 @@ int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int 
     int st;
     const size_t field = (size_t)M * mm * mm;
     if ((st = ensure_buf(L.prods, L.prods_bytes, 6 * field * sizeof(d2v)))) return st;
-    if (X == 192 && M <= 64) {   // the x-transforms as 64-point FFTs across DPP rows
+    // X = 192 and M <= 64: 64-point FFTs across DPP rows (62 us at 129^2 x 64 modes against 83 of
+    // k_xprod_fft); other even X of factors 2, 3 and 5: FFTs through LDS; the remaining sizes (X with
+    // another factor) and the smallest grids (M X <= 1024: 13.5 us at 33^2 x 16 modes, mgalx 48, against
+    // 14.0; at 32 x 96 it is 38 against 26) as dense transforms where those are built, else rocFFT.
+    if (X == 192 && M <= 64) {
         if (!L.xlane) {
             std::vector<double> tab;
             build_xlane_table(tab);
@@ -1217,6 +1238,14 @@ int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int 
         xa.m = mm; xa.M = M; xa.X = X;
         Timed t(PK_XPROD);
         HIPCHK(launch_xprod_lane(xa, L.xlane, L.stream));
+    } else if (xprod_fft_supported(M, X) && !(dense_x(M, X) && M * X <= 1024)) {
+        if ((st = ensure_xtw(X))) return st;
+        XprodArgs xa{};
+        for (int i = 0; i < 3; ++i) xa.in[i] = in[i];
+        for (int p = 0; p < 6; ++p) xa.out[p] = L.prods + p * field;
+        xa.m = mm; xa.M = M; xa.X = X;
+        Timed t(PK_XPROD);
+        HIPCHK(launch_xprod_fft(xa, L.xtw, L.stream));
     } else if (!dense_x(M, X)) {
         if ((st = xprod_fft(in, L.prods, mm, M, X))) return st;
     } else {
@@ -1311,6 +1340,8 @@ int duct_shutdown_(void)
     free_ptr(L.bscr);
     L.bscr_bytes = 0;
     free_ptr(L.xlane);
+    free_ptr(L.xtw);
+    L.xtw_X = 0;
     free_ptr(L.xdft[0]);
     free_ptr(L.xdft[1]);
     L.xdft_M = L.xdft_X = 0;

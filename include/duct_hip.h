@@ -245,8 +245,8 @@ int duct_helm3d_temp_dev_(const duct_devptr_t *rhs, const duct_devptr_t *sol, co
  * hold advection3d of the previous substep's velocity on entry (read when krk > 1)
  * and of this substep's input velocity on exit.  dpdx is the caller's driving
  * gradient (get_dpdx, operators.F:2478-2522: -fnu dpval(aspect)); 0 for none.
- * The advection needs an even mgalx >= 3 nmodes (dense x-DFTs up to 64 modes and
- * 192 points, rocFFT past that).  Both bounds must be set up for m.               */
+ * The advection needs an even mgalx >= 3 nmodes (see duct_advection_dev_).  Both
+ * bounds must be set up for m.                                                     */
 int duct_rk3_substep_dev_(const duct_devptr_t *u, const duct_devptr_t *v, const duct_devptr_t *w,
                           const duct_devptr_t *p, const duct_devptr_t *adv1, const duct_devptr_t *adv2,
                           const duct_devptr_t *adv3, const int *m, const int *nmodes, const int *mgalx,
@@ -286,7 +286,8 @@ int duct_derivx_dev_(const duct_devptr_t *in, const duct_devptr_t *out, const in
  * mult, pack_fftw: src/fourier.F:1-115, src/mult.F) and d/dx = i alp k,
  * d/dy = DC, d/dz = DC / aspect (the collocation form of transyz + derivyz,
  * src/chebyshev.f90).  Needs duct_setup_ for m and an even mgalx >= 3 nmodes
- * (dense x-DFTs up to 64 modes and 192 points, rocFFT past that).  The adv fields must
+ * (one fused kernel for mgalx of factors 2, 3 and 5 up to 2048; other grids as dense
+ * x-DFTs up to 64 modes and 192 points, through rocFFT past that).  The adv fields must
  * not alias u, v, w.  The reference's slip-velocity, CFL and statistics side
  * outputs of advection3d are not computed.                                  */
 int duct_advection_dev_(const duct_devptr_t *u, const duct_devptr_t *v, const duct_devptr_t *w,
