@@ -68,13 +68,10 @@ struct DerivyzArgs {
 hipError_t launch_derivyz(const DerivyzArgs& a, hipStream_t st);
 // Chebyshev transform matrices (column-major m x m): fwd = phys -> coefficients, inv = the inverse.
 void build_cheb_transforms(int m, std::vector<double>& fwd, std::vector<double>& inv);
-// The collocation first and second derivative matrices of the m CGL nodes, column-major m x m,
-// correctly rounded from an extended-precision evaluation (the derivative products' matrices).
-void build_colloc_matrices(int m, std::vector<double>& d1, std::vector<double>& d2);
-// The rows y < ceil(m/2) of D (fold1) and of D2 (fold2) with the contraction folded about the
-// centre node: [Dp | Dm] in fragment layout, each (16 ceil(ceil(m/2)/16))^2 (the derivative
-// products of k_cline_fold on the even and odd parts of their input).
-void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2);
+// The rows y < ceil(m/2) of D (fold1), D2 (fold2) and D^T (fold1t) with the contraction folded about
+// the centre node: [Dp | Dm] in fragment layout, each (16 ceil(ceil(m/2)/16))^2, then the centre row
+// (the derivative products of k_lines on the even and odd parts of their input).
+void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2, std::vector<double>& fold1t);
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd);
 
 // Sizes beyond the dense x-DFT kernels: batched rocFFT real transforms (capi.hip) between these

@@ -342,7 +342,9 @@ void build_cheb_transforms(int m, std::vector<double>& fwd, std::vector<double>&
 }
 
 namespace {
-// D and D2 = D D of the m CGL nodes in extended precision (column-major, D[i + k m]).
+// D and D2 = D D of the m CGL nodes in extended precision (column-major, D[i + k m]).  The product of
+// the double-rounded textbook entries loses ~1e-5 relative in second derivatives at m = 129; these
+// matrices, rounded once, reproduce the interpolant's derivatives to ~1e-10 of the rows' scale.
 void colloc_ld(int m, std::vector<long double>& D, std::vector<long double>& D2)
 {
     // D_ik = (c_i / c_k) (-1)^(i+k) / (x_i - x_k), x_j = -cos(pi j / N) (CHQZ (2.4.31), the matrix of
@@ -375,29 +377,15 @@ void colloc_ld(int m, std::vector<long double>& D, std::vector<long double>& D2)
 }
 }  // namespace
 
-void build_colloc_matrices(int m, std::vector<double>& d1, std::vector<double>& d2)
-{
-    // Both rounded once to double. The product of the double-rounded textbook entries loses ~1e-5
-    // relative in second derivatives at m = 129; these matrices reproduce the interpolant's
-    // derivatives to ~1e-10 of the rows' scale.
-    std::vector<long double> D, D2;
-    colloc_ld(m, D, D2);
-    d1.assign((size_t)m * m, 0.0);
-    d2.assign((size_t)m * m, 0.0);
-    for (size_t e = 0; e < (size_t)m * m; ++e) {
-        d1[e] = (double)D[e];
-        d2[e] = (double)D2[e];
-    }
-}
-
 namespace {
-void fold_rows(int m, const std::vector<long double>& A, std::vector<double>& frag)
+void fold_rows(int m, const std::vector<long double>& A, bool odd, std::vector<double>& frag)
 {
-    // Rows y < he of D (or D2) with the contraction folded about the centre:
-    //   Dp(y, k) = D(y, k) + D(y, m-1-k)  (k < ho),  Dp(y, c) = D(y, c)  (odd m, c = ho)
-    //   Dm(y, k) = D(y, k) - D(y, m-1-k)  (k < ho)
-    // each sum formed in extended precision and rounded once; zero-padded to RT 16 rows and KH
-    // columns, in the fragment layout of build_frag_rect, Dp then Dm.
+    // Rows y < he of A (D, D^T: J A J = -A, odd; D2: J A J = A) with the contraction folded about the centre:
+    //   Dp(y, k) = A(y, k) + A(y, m-1-k)  (k < ho),  Dp(y, c) = A(y, c)  (odd m, c = ho)
+    //   Dm(y, k) = A(y, k) - A(y, m-1-k)  (k < ho)
+    // each sum formed in extended precision and rounded once; zero-padded to KH rows and columns, in the
+    // fragment layout of build_frag_rect, Dp then Dm, then the KH entries of the centre row of the one of
+    // the two that is not zero there (Dm for an odd A, Dp for an even one).
     const int he = (m + 1) / 2, ho = m / 2;
     const int KH = (he + 15) / 16 * 16, R = KH;
     std::vector<double> P((size_t)R * KH, 0.0), Mn((size_t)R * KH, 0.0);
@@ -411,18 +399,24 @@ void fold_rows(int m, const std::vector<long double>& A, std::vector<double>& fr
                 P[y + (size_t)k * R] = (double)a;   // the centre column of odd m
             }
         }
-    frag.assign((size_t)2 * R * KH, 0.0);
+    frag.assign((size_t)2 * R * KH + KH, 0.0);
     build_frag_rect(P.data(), R, KH, R, frag.data());
     build_frag_rect(Mn.data(), R, KH, R, frag.data() + (size_t)R * KH);
+    if (he != ho)
+        for (int k = 0; k < he; ++k) frag[(size_t)2 * R * KH + k] = (odd ? Mn : P)[ho + (size_t)k * R];
 }
 }  // namespace
 
-void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2)
+void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2, std::vector<double>& fold1t)
 {
     std::vector<long double> D, D2;
     colloc_ld(m, D, D2);
-    fold_rows(m, D, fold1);
-    fold_rows(m, D2, fold2);
+    fold_rows(m, D, true, fold1);
+    fold_rows(m, D2, false, fold2);
+    std::vector<long double> T((size_t)m * m);
+    for (int j = 0; j < m; ++j)
+        for (int i = 0; i < m; ++i) T[i + (size_t)j * m] = D[j + (size_t)i * m];
+    fold_rows(m, T, true, fold1t);
 }
 
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd)

@@ -23,10 +23,10 @@
 #include "aux.h"
 #include "common.h"
 #include "h5read.h"
+#include "lines.h"
 #include "mixed_fold.h"
 #include "proj.h"
 #include "proj_lp.h"
-#include "rk3.h"
 #include "temp.h"
 #include "shen.h"
 
@@ -124,10 +124,8 @@ struct Lib {
     d2v* rfield = nullptr;                // residual fields of the mixed solve
     size_t rfield_bytes = 0;
     unsigned long long* stats = nullptr;  // residual maxima of the mixed solve
-    double* dcfrag[2] = {nullptr, nullptr}; // DC and DC^T, FP64 fragment layout (derivative products)
     double* tfrag[2] = {nullptr, nullptr};  // Chebyshev transforms phys->cheb, cheb->phys (transyz)
-    double* d2frag = nullptr;             // D2 = DC DC, FP64 fragment layout (laplacian3d)
-    double* dfold[2] = {nullptr, nullptr};  // D and D2 with the contraction folded (build_colloc_folded)
+    double* dfold[3] = {nullptr, nullptr, nullptr};  // D, D2, D^T with the contraction folded (build_colloc_folded)
     d2v* rk = nullptr;                    // Runge-Kutta substep work fields: h1..h3, advnew1..3, phi
     size_t rk_bytes = 0;
     ShenDev shen[2];                      // Shen-Legendre solve, 'd' and 'n'
@@ -1102,27 +1100,35 @@ int ensure_xtw(int X)
     return OK;
 }
 
-// Independent derivative products (y or z, each its own field, matrix, scale and beta) in one
-// launch on the library's stream, with the derivative matrices of duct_setup_ (padded to L.dc_np).
-int cline_run(int mm, int M, std::initializer_list<ClineOp> ops)
+// One launch of derivative sums (lines.hip) on the library's stream.
+int lines_run(int mm, int M, double alp, bool dirz, const LineJob* jobs, int njobs)
 {
-    ClineArgs c{};
-    c.nmodes = M;
-    c.m = mm;
-    c.NP = L.dc_np;
-    for (const ClineOp& o : ops) {
-        if (c.nops == kMaxClineOps) return fail(ERR_ARG, "more than %d derivative products in one launch", kMaxClineOps);
-        c.op[c.nops++] = o;
-    }
+    LinesArgs a{};
+    a.m = mm;
+    a.nmodes = M;
+    a.mode0 = 0;
+    a.alp = alp;
+    a.dirz = dirz;
+    for (int j = 0; j < njobs; ++j) a.job[a.njobs++] = jobs[j];
     Timed t(PK_DERIV);
-    HIPCHK(launch_cline_ops(c, L.stream));
+    HIPCHK(launch_lines(a, L.stream));
     return OK;
 }
 
-// advection3d (operators.F:9-276) of device fields: the x-transforms and the six products in
-// k_xprod, then the nine derivative terms in the order of operators.F:91-272 per output
-// (adv1: uu_x, uv_y, uw_z; adv2: vv_y, uv_x, vw_z; adv3: ww_z, uw_x, vw_y); the caller has
-// checked the sizes.
+// A job's next stage: its products, output and pointwise terms (see lines.h).
+void add_stage(LineJob& j, int& np, std::initializer_list<LineProd> prods, d2v* out,
+               std::initializer_list<LineTerm> terms, LineTerm self = LineTerm{}, double keep = 0.0, double c0 = 0.0)
+{
+    LineStage& s = j.stage[j.nstage++];
+    s.out = out;
+    s.self = self;
+    s.keep = keep;
+    s.c0 = c0;
+    s.nprod = (int)prods.size();
+    for (const LineProd& p : prods) j.prod[np++] = p;
+    for (const LineTerm& t : terms) s.term[s.nterm++] = t;
+}
+
 // The dense x-DFT kernels (k_xprod, k_fourx) cover M % 16 == 0, M <= 64, X % 16 == 0, X <= 192.
 bool dense_x(int M, int X)
 {
@@ -1216,7 +1222,8 @@ int xprod_fft(const d2v* const in[3], d2v* prods, int mm, int M, int X)
     return OK;
 }
 
-int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int X, double alp, double aspect)
+// The x-part of advection3d (operators.F:9-276): the six products' modes into L.prods.
+int xprods_run(const d2v* const in[3], int mm, int M, int X)
 {
     int st;
     const size_t field = (size_t)M * mm * mm;
@@ -1259,27 +1266,30 @@ int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int 
         Timed t(PK_XPROD);
         HIPCHK(launch_xprod(xa, L.stream));
     }
-    // Each output keeps that order of its three terms; the y and z terms run as two grouped
-    // launches of three independent products.
-    const d2v* P[6];
-    for (int p = 0; p < 6; ++p) P[p] = L.prods + p * field;
-    enum { UU, VV, WW, UV, UW, VW };
-    const double* D = L.dfold[0];   // D folded (J D J = -D)
-    const double sz = 1.0 / aspect;
-    {
-        Timed tm(PK_DERIV);
-        HIPCHK(launch_derivx(P[UU], out[0], mm, M, 0, alp, 1.0, 0.0, L.stream));
+    return OK;
+}
+
+// advection3d's derivative terms (operators.F:91-272): component c is d_x X_c + d_y Q_c + d_z R_c of the
+// products uu, vv, ww, uv, uw, vw.
+enum { UU, VV, WW, UV, UW, VW };
+constexpr int kAdvX[3] = {UU, UV, UW}, kAdvY[3] = {UV, VV, VW}, kAdvZ[3] = {UW, VW, WW};
+
+int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int X, double alp, double aspect)
+{
+    int st;
+    if ((st = xprods_run(in, mm, M, X))) return st;
+    const size_t field = (size_t)M * mm * mm;
+    LineJob jy[3]{}, jz[3]{};
+    for (int c = 0; c < 3; ++c) {
+        int np = 0;
+        add_stage(jy[c], np, {{L.prods + kAdvY[c] * field, L.dfold[0], 1.0, 1}}, out[c],
+                  {{L.prods + kAdvX[c] * field, 0.0, 0.0, 1.0}});
+        np = 0;
+        add_stage(jz[c], np, {{L.prods + kAdvZ[c] * field, L.dfold[0], 1.0 / aspect, 1}}, out[c],
+                  {{out[c], 1.0, 0.0, 0.0}});
     }
-    if ((st = cline_run(mm, M, {{P[UV], out[0], D, 1.0, 1.0, 0, -1}, {P[VV], out[1], D, 1.0, 0.0, 0, -1},
-                                {P[WW], out[2], D, sz, 0.0, 1, -1}})))
-        return st;
-    {
-        Timed tm(PK_DERIV);
-        HIPCHK(launch_derivx(P[UV], out[1], mm, M, 0, alp, 1.0, 1.0, L.stream));
-        HIPCHK(launch_derivx(P[UW], out[2], mm, M, 0, alp, 1.0, 1.0, L.stream));
-    }
-    return cline_run(mm, M, {{P[UW], out[0], D, sz, 1.0, 1, -1}, {P[VW], out[1], D, sz, 1.0, 1, -1},
-                             {P[VW], out[2], D, 1.0, 1.0, 0, -1}});
+    if ((st = lines_run(mm, M, alp, false, jy, 3))) return st;
+    return lines_run(mm, M, alp, true, jz, 3);
 }
 
 }  // namespace
@@ -1321,13 +1331,9 @@ int duct_shutdown_(void)
     for (auto& p : L.hfield) free_ptr(p);
     free_ptr(L.rfield);
     free_ptr(L.stats);
-    free_ptr(L.dcfrag[0]);
-    free_ptr(L.dcfrag[1]);
     free_ptr(L.tfrag[0]);
     free_ptr(L.tfrag[1]);
-    free_ptr(L.d2frag);
-    free_ptr(L.dfold[0]);
-    free_ptr(L.dfold[1]);
+    for (auto& d : L.dfold) free_ptr(d);
     L.dc_m = L.dc_np = 0;
     free_ptr(L.rk);
     L.rk_bytes = 0;
@@ -1487,19 +1493,10 @@ int duct_setup_(const char* bound, const int* m_, const double* P, const double*
         build_frag(T.data(), n, n, NP, bwd.data());
         if ((st = up(B.AbwdT, bwd.data(), bwd.size()))) return st;
     }
-    {   // collocation derivative matrices of the derivative products (DC, DC^T, D2), padded to a
-        // multiple of 16: built here from m in extended precision, not from the caller's DC
+    {   // the Chebyshev transforms (transyz), padded to a multiple of 16, and the derivative matrices of
+        // the derivative products: built here from m in extended precision, not from the caller's DC
         const int MP = (m + 15) / 16 * 16;
-        std::vector<double> f((size_t)MP * MP), T((size_t)m * m), d1, d2;
-        build_colloc_matrices(m, d1, d2);
-        free_ptr(L.dcfrag[0]);
-        free_ptr(L.dcfrag[1]);
-        build_frag(d1.data(), m, m, MP, f.data());
-        if ((st = up(L.dcfrag[0], f.data(), f.size()))) return st;
-        for (int j = 0; j < m; ++j)
-            for (int i = 0; i < m; ++i) T[i + (size_t)j * m] = d1[j + (size_t)i * m];
-        build_frag(T.data(), m, m, MP, f.data());
-        if ((st = up(L.dcfrag[1], f.data(), f.size()))) return st;
+        std::vector<double> f((size_t)MP * MP);
         std::vector<double> tf, ti;
         build_cheb_transforms(m, tf, ti);
         free_ptr(L.tfrag[0]);
@@ -1508,17 +1505,13 @@ int duct_setup_(const char* bound, const int* m_, const double* P, const double*
         if ((st = up(L.tfrag[0], f.data(), f.size()))) return st;
         build_frag(ti.data(), m, m, MP, f.data());
         if ((st = up(L.tfrag[1], f.data(), f.size()))) return st;
-        // D2 = DC DC (pseudomat.f90:110), the full second-derivative matrix of laplacian3d
-        free_ptr(L.d2frag);
-        build_frag(d2.data(), m, m, MP, f.data());
-        if ((st = up(L.d2frag, f.data(), f.size()))) return st;
-        {   // the same products in half the work (k_cline_fold)
-            std::vector<double> f1, f2;
-            build_colloc_folded(m, f1, f2);
-            free_ptr(L.dfold[0]);
-            free_ptr(L.dfold[1]);
-            if ((st = up(L.dfold[0], f1.data(), f1.size()))) return st;
-            if ((st = up(L.dfold[1], f2.data(), f2.size()))) return st;
+        {   // D, D2 and D^T for the products in half the work (k_lines)
+            std::vector<double> f[3];
+            build_colloc_folded(m, f[0], f[1], f[2]);
+            for (int i = 0; i < 3; ++i) {
+                free_ptr(L.dfold[i]);
+                if ((st = up(L.dfold[i], f[i].data(), f[i].size()))) return st;
+            }
         }
         L.dc_m = m;
         L.dc_np = MP;
@@ -2075,7 +2068,7 @@ int duct_advection_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const du
     if (X % 2 || X < 3 * M)
         return fail(ERR_ARG, "advection needs an even mgalx >= 3 nmodes (the 3/2 rule; got %d, %d)", M, X);
     if (!(*aspect > 0.0)) return fail(ERR_ARG, "aspect must be positive");
-    if (!L.dcfrag[0] || !L.dfold[0] || L.dc_m != mm)
+    if (!L.dfold[0] || L.dc_m != mm)
         return fail(ERR_NOT_SETUP, "no collocation matrix for m=%d (duct_setup_ builds it)", mm);
     const d2v* vin[3] = {(const d2v*)in[0], (const d2v*)in[1], (const d2v*)in[2]};
     d2v* vout[3] = {(d2v*)out[0], (d2v*)out[1], (d2v*)out[2]};
@@ -2156,19 +2149,16 @@ int duct_colloc_deriv_dev_(const duct_devptr_t* in, const duct_devptr_t* out, co
     int st = ensure_init();
     if (st) return st;
     if ((st = check_common(*m, *nmodes))) return st;
-    if (!L.dcfrag[0] || L.dc_m != *m)
+    if (!L.dfold[0] || L.dc_m != *m)
         return fail(ERR_NOT_SETUP, "no collocation matrix for m=%d (duct_setup_ builds it)", *m);
-    CollocArgs a{};
-    a.g.nf = 1; a.g.nmodes = *nmodes; a.g.m = *m; a.g.n = *m - 2;
-    a.g.in[0] = (const d2v*)*in;
-    a.g.out[0] = (d2v*)*out;
-    a.Dfrag = L.dcfrag[*trans ? 1 : 0];
-    a.NP = L.dc_np;
-    a.scal = *scal;
-    a.beta = *beta;
-    Timed t(PK_DERIV);
-    HIPCHK(launch_colloc(*cdir == 'y' ? CL_DY : CL_DZ, a, L.stream));
-    return OK;
+    LineJob j{};
+    int np = 0;
+    add_stage(j, np, {{(const d2v*)*in, L.dfold[*trans ? 2 : 0], *scal, 1}}, (d2v*)*out, {});
+    if (*beta != 0.0) {
+        j.stage[0].nterm = 1;
+        j.stage[0].term[0] = LineTerm{(const d2v*)*out, *beta, 0.0, 0.0};
+    }
+    return lines_run(*m, *nmodes, 0.0, *cdir == 'z', &j, 1);
 }
 
 int duct_derivx_dev_(const duct_devptr_t* in, const duct_devptr_t* out, const int* m, const int* nmodes,
@@ -2223,56 +2213,67 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     const int k = *krk - 1;
     const double a = akkc[k], b = bkkc[k], nu = *fnu, ab = a + b, asp = *aspect;
     const size_t field = (size_t)M * mm * mm;
-    if ((st = ensure_buf(L.rk, L.rk_bytes, 9 * field * sizeof(d2v)))) return st;
+    if ((st = ensure_buf(L.rk, L.rk_bytes, 8 * field * sizeof(d2v)))) return st;
     d2v* h[3] = {L.rk, L.rk + field, L.rk + 2 * field};
-    d2v* advnew[3] = {L.rk + 3 * field, L.rk + 4 * field, L.rk + 5 * field};
+    d2v* advt[3] = {L.rk + 3 * field, L.rk + 4 * field, L.rk + 5 * field};   // the x and y terms of advection3d
     d2v* phi = L.rk + 6 * field;
-    d2v* ty = L.rk + 7 * field;   // the y and z terms of a sum, computed in one launch before the x term
-    d2v* tz = L.rk + 8 * field;
+    d2v* lap = L.rk + 7 * field;                                             // the x and y terms of lap(phi)
     d2v* U[3] = {(d2v*)*u, (d2v*)*v, (d2v*)*w};
     d2v* P = (d2v*)*p;
     d2v* ADV[3] = {(d2v*)*adv1, (d2v*)*adv2, (d2v*)*adv3};
     const double* D1 = L.dfold[0];   // D and D2 folded: J D J = -D, J D2 J = D2
     const double* D2 = L.dfold[1];
-    // (ii) adv(u^{k-1}) into advnew
+    // (ii) the products of adv(u^{k-1})
     const d2v* vin[3] = {U[0], U[1], U[2]};
-    if ((st = advection_run(vin, advnew, mm, M, X, *alp, asp))) return st;
-    // (i), (iii)-(vii): h = -1/(nu b) [-rho adv_old - gam adv + nu a lap(u) + u/dt - (a+b) grad p - (a+b) dpdx]
-    const double s = -1.0 / (nu * b);
-    {
-        Rk3RhsArgs r{};
-        for (int c = 0; c < 3; ++c) {
-            r.u[c] = U[c];
-            r.adv[c] = ADV[c];
-            r.advnew[c] = advnew[c];
-            r.h[c] = h[c];
-        }
-        r.p = P;
-        r.mm = (long)mm * mm;
-        r.nmodes = M;
-        r.mode0 = 0;
-        r.use_old = k > 0;
-        r.alp = *alp;
-        r.s = s;
-        r.rho = rkkc[k];
-        r.gam = gkkc[k];
-        r.clap = nu * a;
-        r.rdt = 1.0 / *dt;
-        r.cp = -ab;
-        r.cdp = -ab * *dpdx;
-        Timed t(PK_DERIV);
-        HIPCHK(launch_rk3_rhs(r, L.stream));
-    }
-    // laplacian3d's y parts, then its z parts, scaled as in (vii); then grad3d's y and z parts of p
+    if ((st = xprods_run(vin, mm, M, X))) return st;
+    // (i)-(vii): adv and h = s [-rho adv_old - gam adv + nu a lap(u) + u/dt - (a+b) grad p - (a+b) dpdx],
+    // s = -1/(nu b).  The y launch leaves the x and y terms of adv in advt (adv_old is still needed) and
+    // everything of h but adv and the z derivatives in h; the z launch completes both.
+    const double s = -1.0 / (nu * b), gam = gkkc[k], rho = rkkc[k];
     const double sy2 = s * nu * a, sz2 = s * nu * a / (asp * asp);
-    if ((st = cline_run(mm, M, {{U[0], h[0], D2, sy2, 1.0, 0, 1}, {U[1], h[1], D2, sy2, 1.0, 0, 1},
-                                {U[2], h[2], D2, sy2, 1.0, 0, 1}})))
-        return st;
-    if ((st = cline_run(mm, M, {{U[0], h[0], D2, sz2, 1.0, 1, 1}, {U[1], h[1], D2, sz2, 1.0, 1, 1},
-                                {U[2], h[2], D2, sz2, 1.0, 1, 1}})))
-        return st;
-    if ((st = cline_run(mm, M, {{P, h[1], D1, -s * ab, 1.0, 0, -1}, {P, h[2], D1, -s * ab / asp, 1.0, 1, -1}})))
-        return st;
+    // Where 3 jobs leave CUs idle, adv and h are jobs of their own (h's z job then repeats adv's product),
+    // which shortens the chain of dependent loads and products of a workgroup.
+    // (33^2 x 16 modes: 9.8 + 12.9 against 13.9 + 13.8 us; 97^2 x 40, 728 workgroups: 32.8 + 41.5 against 31.4 + 31.9.)
+    const bool small = 3L * M * mm < 16 * 256;
+    {
+        LineJob jy[6]{}, jz[6]{};
+        int nj = 3;
+        for (int c = 0; c < 3; ++c) {
+            const d2v* X_c = L.prods + kAdvX[c] * field;
+            const LineProd qy = {L.prods + kAdvY[c] * field, D1, 1.0, 1}, lapy = {U[c], D2, sy2, 0}, dpy = {P, D1, -s * ab, 1};
+            const LineTerm tu = {nullptr, s / *dt, -s * nu * a, 0.0};           // lap's x term and u/dt
+            const LineTerm told = {ADV[c], -s * rho, 0.0, 0.0}, tp = {P, 0.0, 0.0, -s * ab};
+            int np = 0;
+            add_stage(jy[c], np, {qy}, advt[c], {{X_c, 0.0, 0.0, 1.0}});
+            LineJob& jh = small ? jy[3 + c] : jy[c];
+            if (small) np = 0;
+            if (c == 0) add_stage(jh, np, {lapy}, h[c], {tp}, tu, 0.0, -s * ab * *dpdx);
+            else if (c == 1) add_stage(jh, np, {dpy, lapy}, h[c], {}, tu);
+            else add_stage(jh, np, {lapy}, h[c], {}, tu);
+            if (k > 0) {   // rkkc(1) = 0: the first substep reads no old term
+                LineStage& g = jh.stage[jh.nstage - 1];
+                g.term[g.nterm++] = told;
+            }
+            const LineProd lapz = {U[c], D2, sz2, 0}, dpz = {P, D1, -s * ab / asp, 1};
+            const LineTerm th = {h[c], 1.0, 0.0, 0.0}, ta = {advt[c], 1.0, 0.0, 0.0};
+            LineProd rz = {L.prods + kAdvZ[c] * field, D1, 1.0 / asp, 1};
+            np = 0;
+            add_stage(jz[c], np, {rz}, ADV[c], {ta}, LineTerm{}, -gam * s);
+            if (!small) {
+                if (c == 2) add_stage(jz[c], np, {lapz, dpz}, h[c], {th});
+                else add_stage(jz[c], np, {lapz}, h[c], {th});
+            } else {
+                const LineTerm tg = {advt[c], -gam * s, 0.0, 0.0};
+                rz.coef *= -gam * s;
+                np = 0;
+                if (c == 2) add_stage(jz[3 + c], np, {rz, lapz, dpz}, h[c], {th, tg});
+                else add_stage(jz[3 + c], np, {rz, lapz}, h[c], {th, tg});
+            }
+        }
+        if (small) nj = 6;
+        if ((st = lines_run(mm, M, *alp, false, jy, nj))) return st;
+        if ((st = lines_run(mm, M, *alp, true, jz, nj))) return st;
+    }
     // (viii) u*, v*, w*: Dirichlet Helmholtz, alambda = 1/(b nu dt)
     {
         const double helco = 1.0 / (b * nu * *dt);
@@ -2283,12 +2284,14 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     }
     // (ix) div3d(u*, v*, w*) / ((a+b) dt) -> h1
     const double sd = 1.0 / (ab * *dt);
-    // (x + y) + z: the y and z products into ty, tz in one launch, then the x term adds them in
-    // that order (the same rounding as accumulating them into h1 one after the other)
-    if ((st = cline_run(mm, M, {{U[1], ty, D1, sd, 0.0, 0, -1}, {U[2], tz, D1, sd / asp, 0.0, 1, -1}}))) return st;
     {
-        Timed t(PK_DERIV);
-        HIPCHK(launch_xderiv(U[0], h[0], (long)mm * mm, M, 0, 1, *alp, sd, 0.0, ty, tz, L.stream));
+        LineJob jy{}, jz{};
+        int np = 0;
+        add_stage(jy, np, {{U[1], D1, sd, 1}}, h[0], {{U[0], 0.0, 0.0, sd}});
+        np = 0;
+        add_stage(jz, np, {{U[2], D1, sd / asp, 1}}, h[0], {{h[0], 1.0, 0.0, 0.0}});
+        if ((st = lines_run(mm, M, *alp, false, &jy, 1))) return st;
+        if ((st = lines_run(mm, M, *alp, true, &jz, 1))) return st;
     }
     // (x) phi: Neumann Poisson
     {
@@ -2297,20 +2300,22 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
         const double al[1] = {0.0};
         if ((st = solve_fields(1, rhs, sol, "n", al, mm, M, 0, *alp, BND_DIR_ZERO))) return st;
     }
-    // (xi) update_uvwp: rhsphi = (a+b) dt nu lap(phi) -> h1; p += phi - rhsphi; u -= dt (a+b) grad phi.
-    // The y and z parts of lap(phi) and of grad(phi) in one launch: all four read phi only, and the
-    // x term and the p, u update that follow touch neither v nor w.
+    // (xi) update_uvwp (operators.F:503-605): p += phi - (a+b) dt nu lap(phi), u_i -= dt (a+b) d_i phi
     const double sl = ab * *dt * nu, su = -*dt * ab;
-    if ((st = cline_run(mm, M, {{phi, ty, D2, sl, 0.0, 0, 1}, {phi, tz, D2, sl / (asp * asp), 0.0, 1, 1},
-                                {phi, U[1], D1, su, 1.0, 0, -1}, {phi, U[2], D1, su / asp, 1.0, 1, -1}})))
-        return st;
     {
-        Timed t(PK_DERIV);
-        HIPCHK(launch_xderiv(phi, h[0], (long)mm * mm, M, 0, 2, *alp, sl, 0.0, ty, tz, L.stream));
-    }
-    {
-        Timed t(PK_DERIV);
-        HIPCHK(launch_rk3_update(P, U[0], phi, h[0], (long)mm * mm, M, 0, *alp, su, L.stream));
+        // one job reads phi's lines once for lap's and grad's products; two shorter ones where CUs are idle
+        LineJob jy[2]{}, jz[2]{};
+        const int g = small ? 1 : 0;
+        int np = 0, nq = 0;
+        add_stage(jy[0], np, {{phi, D2, sl, 0}}, lap, {}, {nullptr, 0.0, -sl, 0.0});
+        add_stage(jy[g], small ? nq : np, {{phi, D1, su, 1}}, U[1], {{U[1], 1.0, 0.0, 0.0}});
+        np = nq = 0;
+        add_stage(jz[0], np, {{phi, D2, -sl / (asp * asp), 0}}, P, {{P, 1.0, 0.0, 0.0}, {lap, -1.0, 0.0, 0.0}},
+                  {nullptr, 1.0, 0.0, 0.0});
+        add_stage(jz[g], small ? nq : np, {{phi, D1, su / asp, 1}}, U[2], {{U[2], 1.0, 0.0, 0.0}});
+        add_stage(jz[g], small ? nq : np, {}, U[0], {{U[0], 1.0, 0.0, 0.0}}, {nullptr, 0.0, 0.0, su});
+        if ((st = lines_run(mm, M, *alp, false, jy, 1 + g))) return st;
+        if ((st = lines_run(mm, M, *alp, true, jz, 1 + g))) return st;
     }
     return OK;
 }

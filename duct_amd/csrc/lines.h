@@ -1,0 +1,51 @@
+// Derivative sums along y or z on whole complex planes (lines.hip).
+#pragma once
+#include "common.h"
+
+namespace duct {
+
+constexpr int kLineProds = 3;    // matrix products of a job
+constexpr int kLineStages = 3;   // outputs of a job
+constexpr int kLineTerms = 2;    // pointwise terms of an output
+constexpr int kLineJobs = 6;     // jobs of a launch
+constexpr int kLineMaxM = 288;   // 9 row tiles of 16 folded rows
+
+// coef * A u along the launch's direction; mat: A folded (build_colloc_folded); odd: J A J = -A (the
+// first derivative and its transpose), else J A J = A (the second).
+struct LineProd {
+    const d2v* src;
+    const double* mat;
+    double coef;
+    int odd;
+};
+// (cr + crx xa^2) t + ci xa (i t), xa = alp (mode0 + mode) of the point's Fourier mode
+struct LineTerm {
+    const d2v* t;
+    double cr, crx, ci;
+};
+// out = carried + the stage's products + terms + self + c0 (on the real part of Fourier mode 0);
+// carried = keep * out of the job's previous stage.  self: a term on the operand of the stage's last
+// product (of an earlier stage's if it has none), which is at hand (self.t is not read).
+struct LineStage {
+    d2v* out;
+    double keep;                 // factor on out for the next stage
+    double c0;
+    int nprod, nterm;            // products of this stage (the job's next ones), terms
+    LineTerm term[kLineTerms];
+    LineTerm self;
+};
+// A job's stages run in order for each of its lines.  An output may be one of its own stage's terms
+// (read before it is written, at the same point), and no product's source or other job's term.
+struct LineJob {
+    LineProd prod[kLineProds];
+    LineStage stage[kLineStages];
+    int nstage;
+};
+struct LinesArgs {
+    LineJob job[kLineJobs];
+    int njobs, m, nmodes, mode0, dirz;
+    double alp;
+};
+hipError_t launch_lines(const LinesArgs& a, hipStream_t st);
+
+}  // namespace duct

@@ -1,0 +1,357 @@
+// Sums of derivative products along y or z with their pointwise terms, for every plane of a field:
+//   y:  out(y, z) = sum_p c_p sum_k A_p(y, k) u_p(k, z) + pointwise terms
+//   z:  out(y, z) = sum_p c_p sum_k A_p(z, k) u_p(y, k) + pointwise terms
+// (derivyz / transyz applied along y or z, chebyshev.f90:1-540, as dense products with the matrices
+// of the m CGL nodes; derivx, fourier.F:117-188, and the elementwise parts of the Runge-Kutta
+// substep, main1.f90:384-655, as the pointwise terms).  One launch of each direction forms all the
+// derivative sums of a step of the algorithm: the right-hand sides, the divergence, the update.
+//
+// Folding: A commutes with the reflection J of the nodes up to a sign, so with u split along the
+// contraction into ue(k) = (u(k) + u(m-1-k)) / 2 and uo(k) = (u(k) - u(m-1-k)) / 2 a product is two
+// half-size ones, Dp ue and Dm uo, and the sums are kept as their even and odd parts E and O:
+// out(r) = E + O, out(m-1-r) = E - O.  An even matrix adds Dp ue to E and Dm uo to O, an odd one the
+// other way round.  The centre row of odd m is one dot product per line on the vector units: as a
+// 17th row it would cost a whole MFMA row tile (he = 65 rows at m = 129: 5 tiles for 4).
+//
+// Work decomposition: a workgroup owns 16 consecutive lines of the flattened (mode, line) index
+// (the planes of odd m would waste most of a tile each) of one job and has one wave per 16 folded
+// rows: a wave computes one tile of E and of O, re and im, so four accumulators, 122 registers, and
+// 16 waves on a CU that hide each other's loads.  (With the next product's lines loaded under the
+// present one's MFMAs, 158 registers and 12 waves: the same times to 2%.)
+//
+// What bounds it: HBM at the sizes whose fields do not stay in the 256 MB last-level cache.  The y
+// and z launches of a substep's right-hand sides at 129^2 x 64 modes read and write 20 fields' worth
+// of 17 MB each (the y launch's sums go through memory to the z launch) in 87 and 95 us, 3.6-3.8
+// TB/s where a copy reaches 4.4-5.1; at 257^2 x 128 modes 816 and 878 us, 3.2 TB/s with the MFMAs
+// busy half the time.  All derivative and elementwise work of an RK3 step took 1537 us at 129^2 x 64
+// as nine launches per substep and takes 870 us as six; at 257^2 x 128, 12800 and 7500 us.
+//
+#include <algorithm>
+
+#include "lines.h"
+
+namespace duct {
+
+namespace {
+constexpr int kLIT = 4;                          // mirrored pairs of points per thread and product
+
+__device__ __forceinline__ d4v mfma(double a, double b, d4v c)
+{
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+}  // namespace
+
+template <bool DIRZ>
+__global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
+{
+    extern __shared__ __attribute__((aligned(16))) double slab[];   // [ue re, uo re, ue im, uo im][line][k]
+    const int m = a.m, he = (m + 1) / 2, ho = m / 2, KH = (he + 15) / 16 * 16;
+    const int KPE = (he + 7) / 8, KPO = (ho + 7) / 8;               // fragment pairs (8 k) of the two parts
+    const int LDK = 8 * KPE + 1, SL = 16 * LDK;
+    const int nth = blockDim.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, l4 = lane >> 4;
+    // slabs in 8 runs, one per XCD; the jobs of a slab are neighbours (they share inputs)
+    const int total = nslab * a.njobs, per = (total + 7) / 8;
+    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+    const LineJob& job = a.job[id % a.njobs];
+    {   // touch the job's arguments at once: their first reads miss the scalar cache one after the other
+        // otherwise, which is most of a small launch's time
+        constexpr int NW = (sizeof(LineJob) + 63) / 64;
+        const int* w = (const int*)&job;
+        int t[NW];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) t[i] = w[i * 16];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) asm volatile("" : : "s"(t[i]));
+    }
+    const int L0 = id / a.njobs * 16;                               // first line
+    const int nlines = min(16, a.nmodes * m - L0);
+    double* red = slab + 4 * SL;                                    // [wave][line][re, im]
+
+    // element offsets of a line's first point and between its points; y: line (mode, z), z: (mode, y)
+    const size_t mm = (size_t)m * m;
+    const int mode_first = L0 / m;
+    const size_t base0 = (size_t)mode_first * mm;
+    const int lrel0 = L0 - mode_first * m;
+    const float invm = 1.0f / (float)m;
+    auto line_off = [&](int l) -> unsigned {                        // relative to base0
+        const int r = lrel0 + l;
+        if constexpr (!DIRZ) return (unsigned)r * m;                // lines of consecutive planes follow each other
+        const int dm = (int)(((float)r + 0.5f) * invm);             // r < m + 16
+        return (unsigned)dm * (unsigned)mm + (r - dm * m);
+    };
+    const unsigned sk = DIRZ ? m : 1;
+
+    // staging: the thread's mirrored pairs (line, k), k < ho (formed anew for each product: kept, their
+    // offsets would cost the registers of the fourth wave per SIMD)
+    const float invh = 1.0f / (float)ho;
+    auto pair_at = [&](int t, int it, int& l, int& k) -> bool {
+        const int e = t + it * nth, q = (int)(((float)e + 0.5f) * invh);   // e < 16 * 144
+        l = DIRZ ? e & 15 : q;
+        k = DIRZ ? e >> 4 : e - q * ho;
+        return e < 16 * ho;
+    };
+    const bool odd_m = he != ho;
+    const bool cok = tid < nlines;                                  // the thread stages a centre point
+    const unsigned oc = line_off(cok ? tid : 0) + ho * sk;
+
+    for (int e = tid; e < 4 * SL; e += nth) slab[e] = 0.0;          // the padding past he and ho stays zero
+
+    d2v va[kLIT], vb[kLIT], vc = {0.0, 0.0};
+    auto load = [&](const d2v* src) {      // lines past the end read line 0 and count as zero
+        const d2v* U = src + base0;
+        int t = tid;
+        asm volatile("" : "+v"(t));
+#pragma unroll
+        for (int it = 0; it < kLIT; ++it) {
+            int l, k;
+            if (!pair_at(t, it, l, k) || l >= nlines) l = k = 0;
+            const unsigned o = line_off(l);
+            va[it] = U[o + k * sk];
+            vb[it] = U[o + (m - 1 - k) * sk];
+        }
+        if (odd_m) vc = U[oc];
+    };
+    auto store = [&]() {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+#pragma unroll
+        for (int it = 0; it < kLIT; ++it) {
+            int l, k;
+            if (!pair_at(t, it, l, k)) continue;
+            const double f = l < nlines ? 0.5 : 0.0;
+            const d2v e = f * (va[it] + vb[it]), o = f * (va[it] - vb[it]);
+            double* s = slab + l * LDK + k;
+            s[0] = e[0];
+            s[SL] = o[0];
+            s[2 * SL] = e[1];
+            s[3 * SL] = o[1];
+        }
+        if (odd_m && tid < 16) {
+            const double f = cok ? 1.0 : 0.0;
+            slab[tid * LDK + ho] = f * vc[0];
+            slab[2 * SL + tid * LDK + ho] = f * vc[1];
+        }
+    };
+
+    d4v ere = {0.0, 0.0, 0.0, 0.0}, eim = ere, ore = ere, oim = ere;   // E and O of the wave's row tile
+    d2v ctr = {0.0, 0.0};                                              // this thread's share of the centre row
+    int q = 0;
+    for (int s = 0; s < job.nstage; ++s) {
+        const LineStage& st = job.stage[s];
+        for (int pi = 0; pi < st.nprod; ++pi, ++q) {
+            const LineProd& p = job.prod[q];
+            const bool odd = p.odd != 0;
+            const d2v* Fp = (const d2v*)p.mat + (size_t)wave * (KH / 8) * 64 + lane;
+            const d2v* Fm = Fp + (size_t)KH * KH / 2;
+            d2v fp = Fp[0], fm = Fm[0];
+            load(p.src);
+            __syncthreads();                                        // the slab's last readers are done
+            store();
+            __syncthreads();
+            const double coef = p.coef;
+            if (odd) {
+                d4v t = ere; ere = ore; ore = t;
+                t = eim; eim = oim; oim = t;
+            }
+            // one pair of k-steps of 4: ue against Dp and uo against Dm, the next pair's fragments in flight
+            const double* S0 = slab + l16 * LDK + l4;
+            auto pair = [&](int kp, const d2v& cp, const d2v& cm, d2v& np, d2v& nm) {
+                const int kn = kp + 1 < KPE ? kp + 1 : kp;
+                np = Fp[(size_t)kn * 64];
+                nm = Fm[(size_t)kn * 64];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const double* S = S0 + (2 * kp + h) * 4;
+                    const double er = S[0], orr = S[SL], ei = S[2 * SL], oi = S[3 * SL];
+                    const double dp = coef * cp[h], dm = coef * cm[h];
+                    if constexpr (!DIRZ) {
+                        ere = mfma(er, dp, ere);
+                        eim = mfma(ei, dp, eim);
+                        ore = mfma(orr, dm, ore);
+                        oim = mfma(oi, dm, oim);
+                    } else {
+                        ere = mfma(dp, er, ere);
+                        eim = mfma(dp, ei, eim);
+                        ore = mfma(dm, orr, ore);
+                        oim = mfma(dm, oi, oim);
+                    }
+                }
+            };
+            d2v gp, gm;
+            int kp = 0;
+            for (; kp + 1 < KPO; kp += 2) {
+                pair(kp, fp, fm, gp, gm);
+                pair(kp + 1, gp, gm, fp, fm);
+            }
+            if (kp < KPO) {
+                pair(kp, fp, fm, gp, gm);
+                fp = gp;
+            }
+            if (KPE > KPO) {                                        // the even part's last pair (he = ho + 1)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const double* S = S0 + (2 * KPO + h) * 4;
+                    const double er = S[0], ei = S[2 * SL];
+                    const double dp = coef * fp[h];
+                    if constexpr (!DIRZ) {
+                        ere = mfma(er, dp, ere);
+                        eim = mfma(ei, dp, eim);
+                    } else {
+                        ere = mfma(dp, er, ere);
+                        eim = mfma(dp, ei, eim);
+                    }
+                }
+            }
+            if (odd) {
+                d4v t = ere; ere = ore; ore = t;
+                t = eim; eim = oim; oim = t;
+            }
+            if (odd_m) {   // centre row: D2's from ue, D's from uo; k = seg, seg + nth / 16, ...
+                const double* C = p.mat + (size_t)2 * KH * KH;
+                const double* S = slab + (odd ? SL : 0) + l16 * LDK;
+                for (int k = tid >> 4; k < he; k += nth >> 4) {
+                    const double c = coef * C[k];
+                    ctr[0] += c * S[k];
+                    ctr[1] += c * S[2 * SL + k];
+                }
+            }
+        }
+
+        // ---- the stage's output: products and terms.  Lane holds rows r (and m-1-r) of 4 lines (y) or
+        // 4 rows of one line (z): D[i][j] in lane j + 16 (i % 4), element i / 4.
+        if (odd_m) {
+            const d2v c = {ctr[0] + __shfl_xor(ctr[0], 16, 64), ctr[1] + __shfl_xor(ctr[1], 16, 64)};
+            const d2v w = {c[0] + __shfl_xor(c[0], 32, 64), c[1] + __shfl_xor(c[1], 32, 64)};
+            if (l4 == 0) {
+                red[(wave * 16 + l16) * 2] = w[0];
+                red[(wave * 16 + l16) * 2 + 1] = w[1];
+            }
+            __syncthreads();
+        }
+        const bool has_c = odd_m && cok, self = st.self.cr != 0.0 || st.self.crx != 0.0 || st.self.ci != 0.0;
+        d2v cv = {0.0, 0.0};
+        if (has_c) {
+            for (int w = 0; w < nth >> 6; ++w) cv += d2v{red[(w * 16 + tid) * 2], red[(w * 16 + tid) * 2 + 1]};
+        }
+        auto mode_of = [&](int l) { return a.mode0 + mode_first + (int)(((float)(lrel0 + l) + 0.5f) * invm); };
+        const int mc = mode_of(l16);
+        const double xc = a.alp * (double)mc;
+        if (has_c) {
+            for (int j = 0; j < st.nterm; ++j) {
+                const LineTerm& t = st.term[j];
+                const d2v y = t.t[base0 + oc];
+                cv += (t.cr + t.crx * xc * xc) * y + t.ci * xc * d2v{-y[1], y[0]};
+            }
+            if (self) {
+                const d2v y = {slab[tid * LDK + ho], slab[2 * SL + tid * LDK + ho]};
+                cv += (st.self.cr + st.self.crx * xc * xc) * y + st.self.ci * xc * d2v{-y[1], y[0]};
+            }
+            if (mc == 0) cv[0] += st.c0;
+            st.out[base0 + oc] = cv;
+        }
+        // (opaque: the addresses of the outputs are cheap to form and are not kept across the products)
+        int q16 = l16, q4 = l4;
+        asm volatile("" : "+v"(q16), "+v"(q4));
+        // two of the lane's four rows at a time (the registers of all four do not fit 4 waves per SIMD)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            unsigned pa[2], pb[2];
+            bool v[2];
+            int md[2];
+            d2v x1[2], x2[2];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const int e = 2 * h + g, i = 4 * e + q4;
+                const int r = 16 * wave + (DIRZ ? i : q16), l = DIRZ ? q16 : i;
+                v[g] = r < ho && l < nlines;
+                const unsigned o = line_off(v[g] ? l : 0), rr = v[g] ? r : 0;
+                pa[g] = o + rr * sk;
+                pb[g] = o + (m - 1 - rr) * sk;
+                md[g] = mode_of(l);
+                x1[g] = d2v{ere[e] + ore[e], eim[e] + oim[e]};
+                x2[g] = d2v{ere[e] - ore[e], eim[e] - oim[e]};
+            }
+            for (int j = 0; j < st.nterm; ++j) {
+                const LineTerm& t = st.term[j];
+                const d2v* T = t.t + base0;
+                d2v y1[2], y2[2];
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    y1[g] = T[pa[g]];
+                    y2[g] = T[pb[g]];
+                }
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const double xa = a.alp * (double)md[g], cr = t.cr + t.crx * xa * xa, ci = t.ci * xa;
+                    x1[g] += cr * y1[g] + ci * d2v{-y1[g][1], y1[g][0]};
+                    x2[g] += cr * y2[g] + ci * d2v{-y2[g][1], y2[g][0]};
+                }
+            }
+            if (self) {   // the slab still holds the last product's operand
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const int i = 4 * (2 * h + g) + q4, r = 16 * wave + (DIRZ ? i : q16), l = DIRZ ? q16 : i;
+                    const double* S = slab + l * LDK + (r < ho ? r : 0);
+                    const d2v e = {S[0], S[2 * SL]}, o = {S[SL], S[3 * SL]};
+                    const double xa = a.alp * (double)md[g], cr = st.self.cr + st.self.crx * xa * xa, ci = st.self.ci * xa;
+                    const d2v y1 = e + o, y2 = e - o;
+                    x1[g] += cr * y1 + ci * d2v{-y1[1], y1[0]};
+                    x2[g] += cr * y2 + ci * d2v{-y2[1], y2[0]};
+                }
+            }
+            d2v* O = st.out + base0;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const double c0 = md[g] == 0 ? st.c0 : 0.0;
+                x1[g][0] += c0;
+                x2[g][0] += c0;
+                if (v[g]) {
+                    O[pa[g]] = x1[g];
+                    O[pb[g]] = x2[g];
+                }
+                const int e = 2 * h + g;   // the next stage starts from keep times this output
+                const d2v ev = (0.5 * st.keep) * (x1[g] + x2[g]), ov = (0.5 * st.keep) * (x1[g] - x2[g]);
+                ere[e] = ev[0];
+                eim[e] = ev[1];
+                ore[e] = ov[0];
+                oim[e] = ov[1];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ctr = has_c ? st.keep * cv : d2v{0.0, 0.0};
+    }
+}
+
+hipError_t launch_lines(const LinesArgs& a, hipStream_t st)
+{
+    if (a.njobs < 0 || a.njobs > kLineJobs || a.m < kMinM || a.m > kLineMaxM) return hipErrorInvalidValue;
+    for (int j = 0; j < a.njobs; ++j) {
+        const LineJob& J = a.job[j];
+        int np = 0;
+        if (J.nstage < 1 || J.nstage > kLineStages) return hipErrorInvalidValue;
+        for (int s = 0; s < J.nstage; ++s) {
+            const LineStage& S = J.stage[s];
+            if (!S.out || S.nprod < 0 || S.nterm < 0 || S.nterm > kLineTerms) return hipErrorInvalidValue;
+            for (int t = 0; t < S.nterm; ++t)
+                if (!S.term[t].t) return hipErrorInvalidValue;
+            np += S.nprod;
+        }
+        if (np < 1 || np > kLineProds) return hipErrorInvalidValue;
+        for (int p = 0; p < np; ++p)
+            if (!J.prod[p].src || !J.prod[p].mat) return hipErrorInvalidValue;
+    }
+    if (a.njobs == 0 || a.nmodes <= 0) return hipSuccess;
+    const int he = (a.m + 1) / 2, ho = a.m / 2;
+    const int nslab = (int)(((long)a.nmodes * a.m + 15) / 16), waves = (ho + 15) / 16;
+    const size_t lds = ((size_t)4 * 16 * (8 * ((he + 7) / 8) + 1) + (size_t)waves * 32) * sizeof(double);
+    const long total = (long)nslab * a.njobs;
+    const dim3 grid((unsigned)((total + 7) / 8 * 8)), block(64 * waves);
+    if (a.dirz) hipLaunchKernelGGL(k_lines<true>, grid, block, lds, st, a, nslab);
+    else hipLaunchKernelGGL(k_lines<false>, grid, block, lds, st, a, nslab);
+    return hipGetLastError();
+}
+
+}  // namespace duct
