@@ -65,7 +65,7 @@ STATUS = {0: "OK", 1: "DUCT_ERR_ARG", 2: "DUCT_ERR_NOT_SETUP", 3: "DUCT_ERR_HIP"
 
 PROF_CLASSES = ["proj_c2p", "proj_p2p_div", "gauge", "proj_p2p", "proj_p2c", "boundary", "bc_correct",
                 "transpose", "invdiag", "lp_c2p", "lp_p2p_div", "lp_p2p", "lp_p2c", "resid", "deriv", "adjoint",
-                "fold_c2p", "fold_p2p_div", "fold_p2p", "fold_p2c", "xprod", "tridiag", "fold_mid"]
+                "fold_c2p", "fold_p2p_div", "fold_p2p", "fold_p2c", "xprod", "tridiag", "fold_mid", "plane"]
 
 
 class DuctError(RuntimeError):

@@ -25,6 +25,7 @@
 #include "h5read.h"
 #include "lines.h"
 #include "mixed_fold.h"
+#include "plane.h"
 #include "proj.h"
 #include "proj_lp.h"
 #include "temp.h"
@@ -110,7 +111,7 @@ enum ProfKind { PK_C2P = 0, PK_P2P_DIV = 1, PK_GAUGE = 2, PK_P2P = 3, PK_P2C = 4
                 PK_TRANSPOSE = 7, PK_INVDIAG = 8, PK_LP_C2P = 9, PK_LP_P2P_DIV = 10, PK_LP_P2P = 11,
                 PK_LP_P2C = 12, PK_RESID = 13, PK_DERIV = 14, PK_ADJ = 15, PK_F_C2P = 16,
                 PK_F_P2P_DIV = 17, PK_F_P2P = 18, PK_F_P2C = 19, PK_XPROD = 20, PK_TRIDIAG = 21,
-                PK_F_MID = 22 };
+                PK_F_MID = 22, PK_PLANE = 23 };
 
 struct Lib {
     bool init = false;
@@ -458,14 +459,94 @@ int run_group_fold(const FieldGroup& g, int bidx, int bmode)
     return OK;
 }
 
-int run_group_unfolded(const FieldGroup& g, int bidx, int bmode);
+int run_group_unfolded(const FieldGroup& g, int bidx, int bmode, bool lds = true);
 
-int run_group(const FieldGroup& g, int bidx, int bmode)
+// Whole solves with the plane in LDS (plane.hip): fields of both boundary types in one launch.
+struct PlaneLaunch {
+    PlaneArgs a{};
+    PlaneLaunch(const FieldGroup& g, int bmode)
+    {
+        a.nmodes = g.nmodes;
+        a.mode0 = g.mode0;
+        a.my = a.mz = g.m;
+        a.alp = g.alp;
+        a.bmode = bmode;
+    }
+    void add(const FieldGroup& g, int bidx, bool adjoint)
+    {
+        const DevBasis& B = L.basis[bidx];
+        PlaneBasis& b = a.b[bidx];
+        const double* fwd = adjoint ? B.AfwdT : B.Afwd;
+        const double* bwd = adjoint ? B.AbwdT : B.Abwd;
+        b.A[0] = b.A[1] = fwd;
+        b.A[2] = b.A[3] = bwd;
+        b.lamy = b.lamz = B.lam;
+        b.prow = B.prow;
+        b.pcol = B.pcol;
+        b.DC = B.DC;
+        b.AM1 = B.AM1;
+        b.pdiag = B.pdiag;
+        b.wanted = B.wanted;
+        b.gauge = bidx == 1 ? B.gauge : -1;
+        b.NP = B.NP;
+        for (int f = 0; f < g.nf; ++f) {
+            a.in[a.nf] = g.in[f];
+            a.out[a.nf] = g.out[f];
+            a.alambda[a.nf] = g.alambda[f];
+            a.bnd[a.nf++] = bidx;
+        }
+    }
+    int run(int kind)
+    {
+        Timed t(PK_PLANE);
+        HIPCHK(launch_plane(kind, a, L.stream));
+        return OK;
+    }
+};
+
+// A launch of whole solves reads a plane and writes its solution while others are still to be read: a
+// solution may be its own right-hand side but overlap no other field (the projection passes read every
+// right-hand side before they write a solution, so those fields keep them).
+bool plane_fields(std::initializer_list<const FieldGroup*> groups)
 {
-    DevBasis& B = L.basis[bidx];
+    std::vector<std::pair<uintptr_t, uintptr_t>> in, out;
+    long planes = 0;
+    for (const FieldGroup* g : groups) planes += 2L * g->nf * g->nmodes;
+    for (const FieldGroup* g : groups) {
+        if (!plane_supported(g->m, g->m, planes)) return false;
+        const uintptr_t bytes = (uintptr_t)g->nmodes * g->m * g->m * sizeof(d2v);
+        for (int f = 0; f < g->nf; ++f) {
+            in.emplace_back((uintptr_t)g->in[f], (uintptr_t)g->in[f] + bytes);
+            out.emplace_back((uintptr_t)g->out[f], (uintptr_t)g->out[f] + bytes);
+        }
+    }
+    auto meet = [](auto& x, auto& y) { return x.first < y.second && y.first < x.second; };
+    for (size_t i = 0; i < out.size(); ++i)
+        for (size_t j = 0; j < in.size(); ++j) {
+            if (meet(out[i], in[j]) && !(i == j && out[i].first == in[j].first)) return false;
+            if (i != j && meet(out[i], out[j])) return false;
+        }
+    return true;
+}
+
+// Solved without the folded bases.
+bool unfolded_group(const FieldGroup& g, int bidx) { return !(L.basis[bidx].NH > 0 && L.fold > bidx); }
+
+int check_group(const FieldGroup& g, int bidx)
+{
+    const DevBasis& B = L.basis[bidx];
     if (!B.ready) return fail(ERR_NOT_SETUP, "duct_setup_ not called for bound '%c'", bidx ? 'n' : 'd');
     if (g.m != B.m) return fail(ERR_ARG, "m=%d but the '%c' basis was set up for m=%d", g.m, bidx ? 'n' : 'd', B.m);
-    if (!(B.NH > 0 && L.fold > bidx)) return run_group_unfolded(g, bidx, bmode);
+    return OK;
+}
+
+// lds: the unfolded solves may keep their planes in LDS (not beside another group's passes, which then
+// wait for the CUs: 742 against 715 us at 129^2 x 256 modes x 4)
+int run_group(const FieldGroup& g, int bidx, int bmode, bool lds = true)
+{
+    int st0 = check_group(g, bidx);
+    if (st0) return st0;
+    if (unfolded_group(g, bidx)) return run_group_unfolded(g, bidx, bmode, lds);
     // folded, except the low Poisson modes of a Neumann group (kLowXlam)
     const int klow = bidx == 1 ? low_mode_prefix(g) : 0;
     int st;
@@ -475,9 +556,14 @@ int run_group(const FieldGroup& g, int bidx, int bmode)
 }
 
 // The four FP64 passes of solvediag in the unfolded eigenbasis, the gauge, the boundary.
-int run_group_unfolded(const FieldGroup& g, int bidx, int bmode)
+int run_group_unfolded(const FieldGroup& g, int bidx, int bmode, bool lds)
 {
     DevBasis& B = L.basis[bidx];
+    if (lds && plane_fields({&g})) {
+        PlaneLaunch p(g, bmode);
+        p.add(g, bidx, false);
+        return p.run(PLANE_FWD);
+    }
     const int NP = B.NP;
     const long cplx_cols = (long)g.nf * g.nmodes * NP;
     const long planes = (long)g.nf * g.nmodes * 2;
@@ -1037,6 +1123,16 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
             ++G.nf;
         }
     }
+    // Planes that fit LDS: every field of both boundary types in one launch.
+    if ((!g[0].nf || unfolded_group(g[0], 0)) && (!g[1].nf || unfolded_group(g[1], 1)) && plane_fields({&g[0], &g[1]})) {
+        PlaneLaunch p(g[0], dir_bmode);
+        for (int bidx = 0; bidx < 2; ++bidx) {
+            if (!g[bidx].nf) continue;
+            if ((st = check_group(g[bidx], bidx))) return st;
+            p.add(g[bidx], bidx, false);
+        }
+        return p.run(PLANE_FWD);
+    }
     // Both groups present: the Neumann group runs on the side stream, so its latency-bound kernels
     // (k=0 gauge, edges) overlap the Dirichlet group's passes. Not while launches are timed: the
     // per-launch hipEvents would then measure kernels that share the GPU.
@@ -1048,11 +1144,11 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
         }
         HIPCHK(hipEventRecord(L.ev_fork, L.stream));
         HIPCHK(hipStreamWaitEvent(L.side, L.ev_fork, 0));
-        st = run_group(g[0], 0, dir_bmode);
+        st = run_group(g[0], 0, dir_bmode, false);
         int st_side;
         {
             SideLane lane;
-            st_side = run_group(g[1], 1, dir_bmode);
+            st_side = run_group(g[1], 1, dir_bmode, false);
         }
         HIPCHK(hipEventRecord(L.ev_join, L.side));
         HIPCHK(hipStreamWaitEvent(L.stream, L.ev_join, 0));
@@ -1060,7 +1156,7 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
     }
     for (int bidx = 0; bidx < 2; ++bidx) {
         if (g[bidx].nf == 0) continue;
-        st = run_group(g[bidx], bidx, dir_bmode);
+        st = run_group(g[bidx], bidx, dir_bmode, !(g[0].nf && g[1].nf));
         if (st) return st;
     }
     return OK;
@@ -1982,8 +2078,9 @@ int duct_helm3d_adjoint_batch_dev_(const int* nfields, const duct_devptr_t* solb
     int st = ensure_init();
     if (st) return st;
     if ((st = check_common(*m, *nmodes))) return st;
+    FieldGroup gs[2]{};
     for (int bidx = 0; bidx < 2; ++bidx) {
-        FieldGroup g{};
+        FieldGroup& g = gs[bidx];
         g.nmodes = *nmodes; g.mode0 = *ib; g.m = *m; g.n = *m - 2; g.alp = *alp;
         for (int f = 0; f < nf; ++f) {
             const int bi = bound_index(bounds[f]);
@@ -1996,10 +2093,15 @@ int duct_helm3d_adjoint_batch_dev_(const int* nfields, const duct_devptr_t* solb
             g.alambda[g.nf] = alambda[f];
             ++g.nf;
         }
-        if (g.nf == 0) continue;
-        if ((st = run_group_adj(g, bidx))) return st;
     }
-    return OK;
+    const bool in_lds = plane_fields({&gs[0], &gs[1]});   // both boundary types in one launch
+    PlaneLaunch p(gs[0], BND_OUT_ZERO);
+    for (int bidx = 0; bidx < 2; ++bidx) {
+        if (gs[bidx].nf == 0) continue;
+        if ((st = in_lds ? check_group(gs[bidx], bidx) : run_group_adj(gs[bidx], bidx))) return st;
+        if (in_lds) p.add(gs[bidx], bidx, true);
+    }
+    return in_lds ? p.run(PLANE_ADJ) : OK;
 }
 
 int duct_fourx_dev_(const duct_devptr_t* fou, const duct_devptr_t* phys, const int* my, const int* nz,
@@ -2411,6 +2513,24 @@ int duct_helm3d_temp_dev_(const duct_devptr_t* rhs, const duct_devptr_t* sol, co
     if (!T.ready || T.my != *my || T.mz != *mz)
         return fail(ERR_NOT_SETUP, "duct_setup_temp_ not called for my=%d, mz=%d", *my, *mz);
     const int NP = T.NP, ny = *my - 2, nz = *mz - 2, M = *nmodes;
+    if (plane_supported(*my, *mz, 2L * M)) {
+        PlaneArgs pa{};
+        pa.in[0] = (const d2v*)*rhs;
+        pa.out[0] = (d2v*)*sol;
+        pa.alambda[0] = *alambda;
+        pa.nf = 1; pa.nmodes = M; pa.mode0 = *ib; pa.my = *my; pa.mz = *mz; pa.alp = *alp;
+        PlaneBasis& b = pa.b[0];
+        b.A[0] = T.Ayi; b.A[1] = T.Azi; b.A[2] = T.Ay; b.A[3] = T.Az;
+        b.lamy = T.ly; b.lamz = T.lz;
+        b.gauge = -1; b.NP = NP;
+        pa.bcy = (const double*)*bcy;
+        pa.bcz = (const double*)*bcz;
+        pa.vec = T.vec;
+        pa.by1 = T.b[0]; pa.by2 = T.b[1]; pa.bz1 = T.b[2]; pa.bz2 = T.b[3];
+        Timed t(PK_PLANE);
+        HIPCHK(launch_plane(PLANE_WALL, pa, L.stream));
+        return OK;
+    }
     const size_t field = (size_t)M * *my * *mz;
     if ((st = ensure_buf(L.tfield, L.tfield_bytes, field * sizeof(d2v)))) return st;
     const long planes = (long)M * 2;

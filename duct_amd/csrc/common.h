@@ -58,4 +58,14 @@ __host__ __device__ inline double xlambda_of(double alambda, double alp, int imo
     return alambda + xa * xa;
 }
 
+// Workgroup barrier for data that is exchanged through LDS.  __syncthreads also waits for the wave's
+// outstanding loads and stores of global memory: a kernel that stores results or fetches ahead and goes
+// on then waits out their latency at every barrier.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 }  // namespace duct

@@ -148,9 +148,9 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
             const d2v* Fm = Fp + (size_t)KH * KH / 2;
             d2v fp = Fp[0], fm = Fm[0];
             load(p.src);
-            __syncthreads();                                        // the slab's last readers are done
+            lds_barrier();                                        // the slab's last readers are done
             store();
-            __syncthreads();
+            lds_barrier();
             const double coef = p.coef;
             if (odd) {
                 d4v t = ere; ere = ore; ore = t;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
                 red[(wave * 16 + l16) * 2] = w[0];
                 red[(wave * 16 + l16) * 2 + 1] = w[1];
             }
-            __syncthreads();
+            lds_barrier();
         }
         const bool has_c = odd_m && cok, self = st.self.cr != 0.0 || st.self.crx != 0.0 || st.self.ci != 0.0;
         d2v cv = {0.0, 0.0};

@@ -165,7 +165,7 @@ __device__ __forceinline__ void pass_r(d2v* Z, const XfftPass& p, const d2v* tw,
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int s = 0; s < MB; ++s) {
         const int e = tid + s * nth;
@@ -175,7 +175,7 @@ __device__ __forceinline__ void pass_r(d2v* Z, const XfftPass& p, const d2v* tw,
             for (int i = 0; i < r; ++i) out[pad8(dst[s] + i * p.ns)] = v[s][i];
         }
     }
-    __syncthreads();
+    lds_barrier();
 }
 
 template <int PT, bool INV>
@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         }
     }
     clear(T);
-    __syncthreads();
+    lds_barrier();
     for (int i = 0; i < a.ninv; ++i) run_pass<PT, true>(Z, a.inv[i], tw, T, ld, tid, nth);
 
     // ---- the last inverse pass: butterfly j of the lines 2 pr and 2 pr + 1
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         last(Z + (2 * pr) * ld, ua);
         last(Z + (2 * pr + 1) * ld, ub);
     }
-    __syncthreads();
+    lds_barrier();
 
     // ---- w of two lines at a time (lane l holds line l's coefficient, its neighbour the partner's)
 #pragma unroll
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         }
     }
     clear(T >> 1);
-    __syncthreads();
+    lds_barrier();
     for (int i = 0; i < a.ninv; ++i) run_pass<PT, true>(Z, a.inv[i], tw, T >> 1, ld, tid, nth);
     if (own) last(Z + pr * ld, ww);
 
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         // kept in registers across the rounds)
         int tq = tid, jq = j, pq = pr;
         asm volatile("" : "+v"(tq), "+v"(jq), "+v"(pq));
-        __syncthreads();
+        lds_barrier();
         if (own) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -312,7 +312,7 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
                 for (int i = 0; i < R; ++i) out[pad8(jq * R + i)] = z[i];
             }
         }
-        __syncthreads();
+        lds_barrier();
         for (int i = 0; i < a.nfwd; ++i) run_pass<PT, false>(Z, a.fwd[i], tw, T, ld, tq, nth);
         d2v* O0 = a.out[2 * q];
         d2v* O1 = a.out[2 * q + 1];

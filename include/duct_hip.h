@@ -407,7 +407,8 @@ int duct_prof_enable_(const int *on);
  * 7 transpose, 8 invdiag, 9 lp_c2p, 10 lp_p2p_div, 11 lp_p2p, 12 lp_p2c,
  * 13 resid, 14 deriv, 15 adjoint (Neumann boundary adjoint), 16 fold_c2p,
  * 17 fold_p2p_div, 18 fold_p2p, 19 fold_p2c, 20 xprod (advection products), 21 tridiag (Shen),
- * 22 fold_mid (folded passes 2 and 3 on LDS-resident quarters).                                */
+ * 22 fold_mid (folded passes 2 and 3 on LDS-resident quarters), 23 plane (whole solves with the
+ * plane in LDS: unfolded, adjoint and mixed-boundary ones with m - 2 <= 128).                  */
 int duct_prof_read_(const int *nclass, double *ms, int *count);
 
 #ifdef __cplusplus
