@@ -26,6 +26,7 @@ struct ProjShape {
     static constexpr int LDB = KT + 1;                       // LDS column stride (doubles)
     static constexpr int NK = NP / KT;                       // LDS stages
     static constexpr int ROWBLOCKS = NP / MT;
+    static constexpr bool TRIM = NP >= 256;                  // only the 16s of rows, columns and k in use are computed
 };
 
 struct ProjArgs {

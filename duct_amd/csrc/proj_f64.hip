@@ -28,9 +28,20 @@
 // buffered, and shared by the waves of the workgroup.  Each wave accumulates a
 // (TM*16) x 64 tile in 4*TM v4f64 accumulators.
 //
+// Padding.  Up to seven eighths of the products of a padded plane are with its zeros, and the passes are bound by the
+// FP64 matrix cores (busy 71-81% of the time at 257^2; the rest is stage turnaround that neither wave
+// priorities, a barrier every second stage nor reading a stage's data ahead of its products took away).  From
+// NP = 256 on (TRIM) a pass therefore computes only the 16s in use: ceil(kn/16) stages, ceil(kn/16) row tiles
+// spread over the waves (TM or TM - 1 each, the larger share rotated over the SIMDs by block), and
+// ceil(cn/16)*16 columns of each plane.  Solves of 4 fields, all of NP -> the 16s in use: 161^2 x 64
+// 1166 -> 420 us, 200^2 x 96 1760 -> 1105, 225^2 x 64 1185 -> 912, 300^2 x 32 4327 -> 1055,
+// 400^2 x 24 3293 -> 1720; full planes the same (257^2 x 256 4.62 ms, 514^2 x 16 2.19).
+//
 // MFMA lane layout (v_mfma_f64_16x16x4f64, checked by tests/test_gpu_solve.py):
 //   A[i][k] from lane i + 16 k, B[k][j] from lane j + 16 k,
 //   D[i][j] in lane j + 16 (i % 4), element i / 4 (rows interleaved by 4).
+#include <type_traits>
+
 #include "common.h"
 #include "proj.h"
 
@@ -44,11 +55,12 @@ __device__ __forceinline__ int vcol_re(int ql) {
     return (ql >> 5) * 64 + ((ql >> 4) & 1) * 32 + (ql & 15);
 }
 
-template <int NP, int MODE>
+template <int NP, int MODE, int TM>
 __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
 {
     using S = ProjShape<NP>;
-    constexpr int NT = S::NT, TM = S::TM, LDB = S::LDB, NK = S::NK;
+    constexpr int NT = S::NT, LDB = S::LDB;
+    constexpr bool TRIM = S::TRIM;
     constexpr bool CIN = MODE == PROJ_C2P;
     constexpr bool COUT = MODE == PROJ_P2C;
     constexpr bool CPLX = CIN || COUT;
@@ -58,16 +70,26 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
     __shared__ double lam_s[LDIV ? NP : 1];
 
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave % S::WM, wn = wave / S::WM;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = TRIM ? (wave + blockIdx.x) & 3 : wave % S::WM, wn = wave / S::WM;
     const int l16 = lane & 15, l4 = lane >> 4;
-    const long tile = blockIdx.x;
+    const unsigned tile = blockIdx.x;
     const int rowblk = blockIdx.y;
     const FieldGroup& g = a.g;
     const int n = g.n, m = g.m;
     // valid extents: K and output rows kn, columns cn; complex fields (ldf, ., .) of fpl points
     const int kn = a.kn ? a.kn : n, cn = a.cn ? a.cn : n, ldf = a.ldf ? a.ldf : m;
     const size_t fpl = a.ldf ? (size_t)a.fplane : (size_t)m * m;
+    // computed extents: all NP, or (TRIM) the 16s that the pass needs: NK stages of k, n16 columns of each
+    // plane, RT row tiles over the waves, TM or TM - 1 each
+    const int NK = TRIM ? (kn + 15) / 16 : S::NK;
+    const unsigned n16 = TRIM ? (cn + 15) / 16 * 16 : NP;
+    const unsigned ncols = TRIM ? (unsigned)(a.ncols / NP) * n16 : (unsigned)a.ncols;
+    constexpr int NWR = S::WM * S::ROWBLOCKS;   // waves along the rows
+    const int wr = rowblk * S::WM + wm;
+    const int rt_base = TRIM ? NK / NWR : TM, rt_more = TRIM ? NK % NWR : 0;
+    const int ntm = rt_base + (wr < rt_more ? 1 : 0);               // this wave's row tiles, from mt0
+    const int mt0 = wr * rt_base + (wr < rt_more ? wr : rt_more);
 
     // ---------------- B-tile loader geometry ----------------
     // planar source (P2P, P2C): each thread loads DPT consecutive k of one column
@@ -92,14 +114,13 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
     if constexpr (MODE == PROJ_P2P || MODE == PROJ_P2P_DIV || LDIV) {
         const int v = tid / TPC;
         kk0 = (tid % TPC) * DPT;
-        const long c = tile * NT + v;
+        const unsigned c = tile * NT + v, plane = c / n16;
         v_dst = v;
-        src_ok = c < a.ncols;
-        if (src_ok) srcp = a.X + (size_t)c * NP;
+        src_ok = c < ncols;
+        if (src_ok) srcp = a.X + ((size_t)plane * NP + c % n16) * NP;
         if constexpr (LDIV) {
-            const long plane = c / NP;
-            ld_j = (int)(c % NP);
-            const long fm = plane >> 1;
+            ld_j = (int)(c % n16);
+            const unsigned fm = plane >> 1;
             const int f = (int)(fm / g.nmodes), mode = (int)(fm % g.nmodes);
             if (src_ok) ld_xlam = xlambda_of(g.alambda[f], g.alp, g.mode0 + mode);
             if (src_ok && ld_j < cn) ld_lamj = (a.lam2 ? a.lam2 : a.lam)[ld_j];
@@ -112,11 +133,10 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
         const int t = (v & 63) >> 4;
         const int ql = (v >> 6) * 32 + (t >> 1) * 16 + (v & 15);
         const int part = t & 1;
-        const long q = tile * (NT / 2) + ql;
-        src_ok = q < a.ncols;
+        const unsigned q = tile * (NT / 2) + ql;
+        src_ok = q < ncols;
         if (src_ok) {
-            const long fm = q / NP;
-            const int j = (int)(q % NP);
+            const unsigned fm = q / n16, j = q % n16;
             srcp = a.X + ((size_t)(fm * 2 + part) * NP + j) * NP;
         }
     } else {  // C2P
@@ -124,10 +144,10 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
         kk0 = (tid % TPQ) * CPT;
         v_dst = vcol_re(ql);
         v_dst_im = v_dst + 16;
-        const long q = tile * (NT / 2) + ql;
-        if (q < a.ncols) {
-            const long fm = q / NP;
-            const int j = (int)(q % NP);
+        const unsigned q = tile * (NT / 2) + ql;
+        if (q < ncols) {
+            const unsigned fm = q / n16;
+            const int j = (int)(q % n16);
             const int f = (int)(fm / g.nmodes), mode = (int)(fm % g.nmodes);
             src_ok = j < cn;
             zero_im = (g.mode0 + mode) == 0;   // int2d3d.f90:43 skips Im at k=0
@@ -182,75 +202,101 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
         }
     };
 
-    // ---------------- A fragments (global, fragment-major) ----------------
-    const int mt0 = (rowblk * S::MT + wm * S::WR) / 16;
-    const d2v* Ab = (const d2v*)a.Afrag + (size_t)mt0 * (NP / 8) * 64 + lane;
-    d2v acur[TM][2], anext[TM][2];
-    auto load_a = [&](int ks, d2v (&dst)[TM][2]) {
-#pragma unroll
-        for (int mt = 0; mt < TM; ++mt)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) dst[mt][h] = Ab[((size_t)mt * (NP / 8) + ks * 2 + h) * 64];
-    };
-
+    // ---------------- products ----------------
     d4v acc[TM][4];
 #pragma unroll
     for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = d4v{0.0, 0.0, 0.0, 0.0};
 
-    load_b(0);
-    load_a(0, acur);
-    store_b(0, 0);
-    __syncthreads();
-
-    for (int ks = 0; ks < NK; ++ks) {
-        const int buf = ks & 1;
-        if (ks + 1 < NK) {
-            load_b(ks + 1);
-            load_a(ks + 1, anext);
-        }
-        const double* B = Bs[buf];
+    const d2v* Ab = (const d2v*)a.Afrag + (size_t)mt0 * (NP / 8) * 64 + lane;   // fragment-major
+    // the stages with T row tiles of this wave (both bodies pass the same barriers)
+    auto stages = [&](auto tiles) {
+        constexpr int T = decltype(tiles)::value;
+        auto load_a = [&](int ks, d2v (&dst)[T][2]) {
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            double bf[4];
+            for (int mt = 0; mt < T; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) bf[nt] = B[(wn * 64 + nt * 16 + l16) * LDB + kk * 4 + l4];
+                for (int h = 0; h < 2; ++h) dst[mt][h] = Ab[((size_t)mt * (NP / 8) + ks * 2 + h) * 64];
+        };
+        auto mma = [&](const double* B, const d2v (&af)[T][2]) {
 #pragma unroll
-            for (int mt = 0; mt < TM; ++mt) {
-                const double av = acur[mt][kk >> 1][kk & 1];
+            for (int kk = 0; kk < 4; ++kk) {
+                double bf[4];
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bf[nt], acc[mt][nt], 0, 0, 0);
+                for (int nt = 0; nt < 4; ++nt) bf[nt] = B[(wn * 64 + nt * 16 + l16) * LDB + kk * 4 + l4];
+#pragma unroll
+                for (int mt = 0; mt < T; ++mt) {
+                    const double av = af[mt][kk >> 1][kk & 1];
+#pragma unroll
+                    for (int nt = 0; nt < 4; ++nt)
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bf[nt], acc[mt][nt], 0, 0, 0);
+                }
             }
-        }
-        if (ks + 1 < NK) {
-            store_b(buf ^ 1, ks + 1);
-#pragma unroll
-            for (int mt = 0; mt < TM; ++mt) {
-                acur[mt][0] = anext[mt][0];
-                acur[mt][1] = anext[mt][1];
-            }
-        }
+        };
+        d2v a0[T][2], a1[T][2];
+        load_b(0);
+        load_a(0, a0);
+        store_b(0, 0);
         __syncthreads();
-    }
+        if constexpr (TRIM) {
+            // a stage count known at run time: two stages per iteration with the fragment buffers swapped (a
+            // copy at the loop's end would wait for the loads it rotates in), and the loads of the stage
+            // past the last repeat it (under a branch they would be waited for at once)
+            auto stage = [&](int ks, const d2v (&cur)[T][2], d2v (&nxt)[T][2]) {
+                const int kn1 = ks + 1 < NK ? ks + 1 : ks;
+                load_b(kn1);
+                load_a(kn1, nxt);
+                mma(Bs[ks & 1], cur);
+                store_b((ks & 1) ^ 1, kn1);
+                __syncthreads();
+            };
+            int ks = 0;
+            for (; ks + 1 < NK; ks += 2) {
+                stage(ks, a0, a1);
+                stage(ks + 1, a1, a0);
+            }
+            if (ks < NK) mma(Bs[ks & 1], a0);
+        } else {
+            for (int ks = 0; ks < NK; ++ks) {
+                const int buf = ks & 1;
+                if (ks + 1 < NK) {
+                    load_b(ks + 1);
+                    load_a(ks + 1, a1);
+                }
+                mma(Bs[buf], a0);
+                if (ks + 1 < NK) {
+                    store_b(buf ^ 1, ks + 1);
+#pragma unroll
+                    for (int mt = 0; mt < T; ++mt) {
+                        a0[mt][0] = a1[mt][0];
+                        a0[mt][1] = a1[mt][1];
+                    }
+                }
+                __syncthreads();
+            }
+        }
+    };
+    if (!TRIM || ntm == TM) stages(std::integral_constant<int, TM>{});
+    else stages(std::integral_constant<int, TRIM ? TM - 1 : TM>{});
 
     // ---------------- epilogue ----------------
-    const int rbase = rowblk * S::MT + wm * S::WR + l4;
+    const int rbase = mt0 * 16 + l4;
     if constexpr (COUT) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             const int ql = wn * 32 + s * 16 + l16;
-            const long q = tile * (NT / 2) + ql;
-            if (q >= a.ncols) continue;
-            const long fm = q / NP;
-            const int j = (int)(q % NP);
+            const unsigned q = tile * (NT / 2) + ql;
+            if (q >= ncols) continue;
+            const unsigned fm = q / n16;
+            const int j = (int)(q % n16);
             if (j >= cn) continue;
             const int f = (int)(fm / g.nmodes), mode = (int)(fm % g.nmodes);
             const bool zim = (g.mode0 + mode) == 0;
             d2v* out = g.out[f] + (size_t)mode * fpl + (j + 1);
 #pragma unroll
-            for (int mt = 0; mt < TM; ++mt)
+            for (int mt = 0; mt < TM; ++mt) {
+                if (TRIM && mt >= ntm) break;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = rbase + mt * 16 + 4 * r;
@@ -259,6 +305,7 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
                         out[(size_t)(row + 1) * ldf] = v;
                     }
                 }
+            }
         }
     } else {
         // divide epilogue: the row eigenvalues are loaded once, before any store
@@ -275,34 +322,35 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
         }
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
-            long plane;
+            unsigned plane;
             int j;
             bool ok;
             if constexpr (CIN) {
                 const int ql = wn * 32 + (nt >> 1) * 16 + l16;
-                const long q = tile * (NT / 2) + ql;
-                ok = q < a.ncols;
-                plane = (q / NP) * 2 + (nt & 1);
-                j = (int)(q % NP);
+                const unsigned q = tile * (NT / 2) + ql;
+                ok = q < ncols;
+                plane = (q / n16) * 2 + (nt & 1);
+                j = (int)(q % n16);
             } else {
-                const long c = tile * NT + wn * 64 + nt * 16 + l16;
-                ok = c < a.ncols;
-                plane = c / NP;
-                j = (int)(c % NP);
+                const unsigned c = tile * NT + wn * 64 + nt * 16 + l16;
+                ok = c < ncols;
+                plane = c / n16;
+                j = (int)(c % n16);
             }
             if (!ok) continue;
             double* Y = a.Y + (size_t)plane * NP * NP + j;
             double xlam = 0.0, lj = 0.0;
             bool gauge_plane = false;
             if constexpr (MODE == PROJ_P2P_DIV) {
-                const long fm = plane >> 1;
+                const unsigned fm = plane >> 1;
                 const int f = (int)(fm / g.nmodes), mode = (int)(fm % g.nmodes);
                 xlam = xlambda_of(g.alambda[f], g.alp, g.mode0 + mode);
                 gauge_plane = a.gauge >= 0 && fabs(xlam) <= 1.0e-10;
                 lj = j < cn ? a.lam[j] : 0.0;
             }
 #pragma unroll
-            for (int mt = 0; mt < TM; ++mt)
+            for (int mt = 0; mt < TM; ++mt) {
+                if (TRIM && mt >= ntm) break;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = rbase + mt * 16 + 4 * r;
@@ -315,8 +363,24 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
                     }
                     Y[(size_t)row * NP] = v;
                 }
+            }
         }
     }
+}
+
+template <int NP, int TM>
+static hipError_t launch_tm(int mode, const ProjArgs& a, dim3 grid, hipStream_t st)
+{
+    const dim3 block(256);
+    switch (mode) {
+        case PROJ_C2P: hipLaunchKernelGGL((k_proj<NP, PROJ_C2P, TM>), grid, block, 0, st, a); break;
+        case PROJ_P2P: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P, TM>), grid, block, 0, st, a); break;
+        case PROJ_P2P_DIV: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P_DIV, TM>), grid, block, 0, st, a); break;
+        case PROJ_P2C: hipLaunchKernelGGL((k_proj<NP, PROJ_P2C, TM>), grid, block, 0, st, a); break;
+        case PROJ_P2P_LDIV: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P_LDIV, TM>), grid, block, 0, st, a); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 template <int NP>
@@ -325,18 +389,24 @@ static hipError_t launch_np(int mode, const ProjArgs& a, hipStream_t st)
     using S = ProjShape<NP>;
     const bool cplx = mode == PROJ_C2P || mode == PROJ_P2C;
     const long per = cplx ? S::NT / 2 : S::NT;
-    const long tiles = (a.ncols + per - 1) / per;
+    const int kn = a.kn ? a.kn : a.g.n, cn = a.cn ? a.cn : a.g.n;
+    const int k16 = (kn + 15) / 16, c16 = (cn + 15) / 16;   // 16s in use
+    const long ncols = S::TRIM ? a.ncols / NP * c16 * 16 : a.ncols;
+    if (a.ncols < 0 || a.ncols >= 1L << 31) return hipErrorInvalidValue;   // 32-bit column indices
+    const long tiles = (ncols + per - 1) / per;
     if (tiles <= 0) return hipSuccess;
-    dim3 grid((unsigned)tiles, S::ROWBLOCKS), block(256);
-    switch (mode) {
-        case PROJ_C2P: hipLaunchKernelGGL((k_proj<NP, PROJ_C2P>), grid, block, 0, st, a); break;
-        case PROJ_P2P: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P>), grid, block, 0, st, a); break;
-        case PROJ_P2P_DIV: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P_DIV>), grid, block, 0, st, a); break;
-        case PROJ_P2C: hipLaunchKernelGGL((k_proj<NP, PROJ_P2C>), grid, block, 0, st, a); break;
-        case PROJ_P2P_LDIV: hipLaunchKernelGGL((k_proj<NP, PROJ_P2P_LDIV>), grid, block, 0, st, a); break;
-        default: return hipErrorInvalidValue;
+    const dim3 grid((unsigned)tiles, S::ROWBLOCKS);
+    if constexpr (S::TRIM) {   // the most row tiles that a wave owns, over the waves of all row blocks
+        constexpr int nw = S::WM * S::ROWBLOCKS;
+        switch ((k16 + nw - 1) / nw) {
+            case 1:
+            case 2: return launch_tm<NP, 2>(mode, a, grid, st);
+            case 3: return launch_tm<NP, 3>(mode, a, grid, st);
+            case 4: return launch_tm<NP, 4>(mode, a, grid, st);
+            default: return hipErrorInvalidValue;
+        }
     }
-    return hipGetLastError();
+    return launch_tm<NP, S::TM>(mode, a, grid, st);
 }
 
 hipError_t launch_proj(int NP, int mode, const ProjArgs& a, hipStream_t st)
