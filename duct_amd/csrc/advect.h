@@ -72,6 +72,8 @@ void build_cheb_transforms(int m, std::vector<double>& fwd, std::vector<double>&
 // the centre node: [Dp | Dm] in fragment layout, each (16 ceil(ceil(m/2)/16))^2, then the centre row
 // (the derivative products of k_lines on the even and odd parts of their input).
 void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2, std::vector<double>& fold1t);
+// D and D2 themselves, column-major (k_sums)
+void build_colloc_full(int m, std::vector<double>& full1, std::vector<double>& full2);
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd);
 
 // Sizes beyond the dense x-DFT kernels: batched rocFFT real transforms (capi.hip) between these

@@ -419,6 +419,14 @@ void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>&
     fold_rows(m, T, true, fold1t);
 }
 
+void build_colloc_full(int m, std::vector<double>& full1, std::vector<double>& full2)
+{
+    std::vector<long double> D, D2;
+    colloc_ld(m, D, D2);
+    full1.assign(D.begin(), D.end());
+    full2.assign(D2.begin(), D2.end());
+}
+
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd)
 {
     const int Q = 2 * M;

@@ -127,6 +127,7 @@ struct Lib {
     unsigned long long* stats = nullptr;  // residual maxima of the mixed solve
     double* tfrag[2] = {nullptr, nullptr};  // Chebyshev transforms phys->cheb, cheb->phys (transyz)
     double* dfold[3] = {nullptr, nullptr, nullptr};  // D, D2, D^T with the contraction folded (build_colloc_folded)
+    double* dfull[2] = {nullptr, nullptr};  // D, D2 in fragments, for m <= kSumMaxM (build_colloc_full)
     d2v* rk = nullptr;                    // Runge-Kutta substep work fields: h1..h3, advnew1..3, phi
     size_t rk_bytes = 0;
     ShenDev shen[2];                      // Shen-Legendre solve, 'd' and 'n'
@@ -1225,6 +1226,40 @@ void add_stage(LineJob& j, int& np, std::initializer_list<LineProd> prods, d2v* 
     for (const LineTerm& t : terms) s.term[s.nterm++] = t;
 }
 
+// One launch of derivative sums along both directions (k_sums).
+int sums_run(int mm, int M, double alp, const SumJob* jobs, int njobs)
+{
+    SumArgs a{};
+    a.m = mm;
+    a.nmodes = M;
+    a.alp = alp;
+    for (int j = 0; j < njobs; ++j) a.job[a.njobs++] = jobs[j];
+    Timed t(PK_DERIV);
+    HIPCHK(launch_sums(a, L.stream));
+    return OK;
+}
+
+// A job's next output: its products along y and z and its pointwise terms (see lines.h).
+void add_sum(SumJob& j, std::initializer_list<SumProd> py, std::initializer_list<SumProd> pz, d2v* out,
+             std::initializer_list<LineTerm> terms, double keep = 0.0, double c0 = 0.0)
+{
+    SumStage& s = j.stage[j.nstage++];
+    s.out = out;
+    s.keep = keep;
+    s.c0 = c0;
+    int d = 0;
+    for (const auto& list : {py, pz}) {
+        int np = 0;
+        for (int t = 0; t + 1 < j.nstage; ++t) np += j.stage[t].nprod[d];
+        for (const SumProd& p : list) j.prod[d][np++] = p;
+        s.nprod[d++] = (int)list.size();
+    }
+    for (const LineTerm& t : terms)
+        if (t.t) s.term[s.nterm++] = t;
+    for (auto& p : j.prod)   // a direction without products reads a valid address in vain
+        if (!p[0].src) p[0] = {s.term[0].t, L.dfull[0], 0.0};
+}
+
 // The dense x-DFT kernels (k_xprod, k_fourx) cover M % 16 == 0, M <= 64, X % 16 == 0, X <= 192.
 bool dense_x(int M, int X)
 {
@@ -1375,6 +1410,13 @@ int advection_run(const d2v* const in[3], d2v* const out[3], int mm, int M, int 
     int st;
     if ((st = xprods_run(in, mm, M, X))) return st;
     const size_t field = (size_t)M * mm * mm;
+    if (sums_supported(mm, M)) {
+        SumJob js[3]{};
+        for (int c = 0; c < 3; ++c)
+            add_sum(js[c], {{L.prods + kAdvY[c] * field, L.dfull[0], 1.0}}, {{L.prods + kAdvZ[c] * field, L.dfull[0], 1.0 / aspect}},
+                    out[c], {{L.prods + kAdvX[c] * field, 0.0, 0.0, 1.0}});
+        return sums_run(mm, M, alp, js, 3);
+    }
     LineJob jy[3]{}, jz[3]{};
     for (int c = 0; c < 3; ++c) {
         int np = 0;
@@ -1430,6 +1472,7 @@ int duct_shutdown_(void)
     free_ptr(L.tfrag[0]);
     free_ptr(L.tfrag[1]);
     for (auto& d : L.dfold) free_ptr(d);
+    for (auto& d : L.dfull) free_ptr(d);
     L.dc_m = L.dc_np = 0;
     free_ptr(L.rk);
     L.rk_bytes = 0;
@@ -1607,6 +1650,15 @@ int duct_setup_(const char* bound, const int* m_, const double* P, const double*
             for (int i = 0; i < 3; ++i) {
                 free_ptr(L.dfold[i]);
                 if ((st = up(L.dfold[i], f[i].data(), f[i].size()))) return st;
+            }
+        }
+        for (auto& d : L.dfull) free_ptr(d);
+        if (m <= kSumMaxM) {   // D and D2 as they are (k_sums)
+            std::vector<double> d[2];
+            build_colloc_full(m, d[0], d[1]);
+            for (int i = 0; i < 2; ++i) {
+                build_frag(d[i].data(), m, m, MP, f.data());
+                if ((st = up(L.dfull[i], f.data(), f.size()))) return st;
             }
         }
         L.dc_m = m;
@@ -2336,8 +2388,24 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     // Where 3 jobs leave CUs idle, adv and h are jobs of their own (h's z job then repeats adv's product),
     // which shortens the chain of dependent loads and products of a workgroup.
     // (33^2 x 16 modes: 9.8 + 12.9 against 13.9 + 13.8 us; 97^2 x 40, 728 workgroups: 32.8 + 41.5 against 31.4 + 31.9.)
-    const bool small = 3L * M * mm < 16 * 256;
-    {
+    const bool small = 3L * M * mm < 16 * 256, sums = sums_supported(mm, M);
+    if (sums) {
+        const double* F1 = L.dfull[0];
+        const double* F2 = L.dfull[1];
+        SumJob js[3]{};
+        for (int c = 0; c < 3; ++c) {
+            const SumProd lapy = {U[c], F2, sy2}, lapz = {U[c], F2, sz2};
+            const SumProd dpy = {P, F1, -s * ab}, dpz = {P, F1, -s * ab / asp};
+            const LineTerm tu = {U[c], s / *dt, -s * nu * a, 0.0}, tp = {P, 0.0, 0.0, -s * ab};
+            const LineTerm told = {k > 0 ? ADV[c] : nullptr, -s * rho, 0.0, 0.0};   // (the first substep reads no old term)
+            add_sum(js[c], {{L.prods + kAdvY[c] * field, F1, 1.0}}, {{L.prods + kAdvZ[c] * field, F1, 1.0 / asp}}, ADV[c],
+                    {{L.prods + kAdvX[c] * field, 0.0, 0.0, 1.0}});
+            if (c == 0) add_sum(js[c], {lapy}, {lapz}, h[c], {tp, tu, told}, -gam * s, -s * ab * *dpdx);
+            else if (c == 1) add_sum(js[c], {lapy, dpy}, {lapz}, h[c], {tu, told}, -gam * s);
+            else add_sum(js[c], {lapy}, {lapz, dpz}, h[c], {tu, told}, -gam * s);
+        }
+        if ((st = sums_run(mm, M, *alp, js, 3))) return st;
+    } else {
         LineJob jy[6]{}, jz[6]{};
         int nj = 3;
         for (int c = 0; c < 3; ++c) {
@@ -2386,7 +2454,11 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     }
     // (ix) div3d(u*, v*, w*) / ((a+b) dt) -> h1
     const double sd = 1.0 / (ab * *dt);
-    {
+    if (sums) {
+        SumJob j{};
+        add_sum(j, {{U[1], L.dfull[0], sd}}, {{U[2], L.dfull[0], sd / asp}}, h[0], {{U[0], 0.0, 0.0, sd}});
+        if ((st = sums_run(mm, M, *alp, &j, 1))) return st;
+    } else {
         LineJob jy{}, jz{};
         int np = 0;
         add_stage(jy, np, {{U[1], D1, sd, 1}}, h[0], {{U[0], 0.0, 0.0, sd}});
@@ -2404,7 +2476,14 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     }
     // (xi) update_uvwp (operators.F:503-605): p += phi - (a+b) dt nu lap(phi), u_i -= dt (a+b) d_i phi
     const double sl = ab * *dt * nu, su = -*dt * ab;
-    {
+    if (sums) {
+        SumJob js[3]{};
+        add_sum(js[0], {{phi, L.dfull[1], -sl}}, {{phi, L.dfull[1], -sl / (asp * asp)}}, P, {{P, 1.0, 0.0, 0.0}, {phi, 1.0, sl, 0.0}});
+        add_sum(js[1], {{phi, L.dfull[0], su}}, {}, U[1], {{U[1], 1.0, 0.0, 0.0}});
+        add_sum(js[1], {}, {}, U[0], {{U[0], 1.0, 0.0, 0.0}, {phi, 0.0, 0.0, su}});
+        add_sum(js[2], {}, {{phi, L.dfull[0], su / asp}}, U[2], {{U[2], 1.0, 0.0, 0.0}});
+        if ((st = sums_run(mm, M, *alp, js, 3))) return st;
+    } else {
         // one job reads phi's lines once for lap's and grad's products; two shorter ones where CUs are idle
         LineJob jy[2]{}, jz[2]{};
         const int g = small ? 1 : 0;

@@ -48,4 +48,40 @@ struct LinesArgs {
 };
 hipError_t launch_lines(const LinesArgs& a, hipStream_t st);
 
+// The same sums along both directions in one launch, for small planes (k_sums).
+constexpr int kSumProds = 3;     // products of a job per direction
+constexpr int kSumTerms = 3;     // pointwise terms of an output
+constexpr int kSumStages = 2;    // outputs of a job
+constexpr int kSumJobs = 3;      // jobs of a launch
+constexpr int kSumMaxM = 64;
+
+// coef * A u along the list's direction; mat: A in fragments of 16 rows (build_frag of build_colloc_full)
+struct SumProd {
+    const d2v* src;
+    const double* mat;
+    double coef;
+};
+// out = keep * the previous stage's out + the stage's products + terms + c0 (on the real part of Fourier
+// mode 0).  The terms of a job are read before its outputs are written, at the same point; no output is a
+// product's source or another job's term.
+struct SumStage {
+    d2v* out;
+    double keep, c0;
+    int nprod[2], nterm;         // products along y, z (the job's next ones), terms
+    LineTerm term[kSumTerms];
+};
+struct SumJob {
+    SumProd prod[2][kSumProds];  // along y, along z
+    SumStage stage[kSumStages];
+    int nstage;
+};
+struct SumArgs {
+    SumJob job[kSumJobs];
+    int njobs, m, nmodes;
+    double alp;
+};
+// planes small and few enough for k_sums
+bool sums_supported(int m, int nmodes);
+hipError_t launch_sums(const SumArgs& a, hipStream_t st);
+
 }  // namespace duct

@@ -27,6 +27,7 @@
 // as nine launches per substep and takes 870 us as six; at 257^2 x 128, 12800 and 7500 us.
 //
 #include <algorithm>
+#include <type_traits>
 
 #include "lines.h"
 
@@ -351,6 +352,198 @@ hipError_t launch_lines(const LinesArgs& a, hipStream_t st)
     const dim3 grid((unsigned)((total + 7) / 8 * 8)), block(64 * waves);
     if (a.dirz) hipLaunchKernelGGL(k_lines<true>, grid, block, lds, st, a, nslab);
     else hipLaunchKernelGGL(k_lines<false>, grid, block, lds, st, a, nslab);
+    return hipGetLastError();
+}
+
+// ---- small planes: both directions in one launch ----------------------------------------------
+// A small grid's step is a chain of launches that are latency: arguments, loads, a few products, stores.  Here
+// a workgroup owns one 16 x 16 tile of a job's outputs on one mode, its first wave the products along y, its
+// second those along z, with the operands straight from memory into registers (the loads of all products are
+// issued before the first product; the planes are a few KB and come from the caches), no staging and one
+// barrier, where the second wave's sums join the first's.  Nothing is folded: at these sizes the products are
+// a third of a workgroup's time.  A 33^2 x 16 step of 27 launches took 251 us, of these 18 y and z launches;
+// with 9 of k_sums it takes 141 us.
+template <int KP, int NPR>
+__global__ __launch_bounds__(128) void k_sums(SumArgs a)
+{
+    __shared__ d2v ex[kSumStages][4][64];
+    const int m = a.m, nt = (m + 15) / 16;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, l4 = lane >> 4;
+    // modes in 8 runs, one per XCD; the tiles and jobs of a mode are neighbours (they share inputs)
+    const int total = a.njobs * a.nmodes * nt * nt, per = (total + 7) / 8;
+    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+    const int ty = id % nt, tz = id / nt % nt, jm = id / (nt * nt), mode = jm / a.njobs;
+    const SumJob& job = a.job[jm % a.njobs];
+    {   // touch the job's arguments at once (their first reads miss the scalar cache one after the other otherwise)
+        constexpr int NW = (sizeof(SumJob) + 63) / 64;
+        const int* w = (const int*)&job;
+        int t[NW];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) t[i] = w[min(i * 16, (int)sizeof(SumJob) / 4 - 1)];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) asm volatile("" : : "s"(t[i]));
+    }
+    const size_t base = (size_t)mode * m * m;
+    const int z16 = 16 * tz, y16 = 16 * ty;
+    d4v re[kSumStages], im[kSumStages];
+#pragma unroll
+    for (int s = 0; s < kSumStages; ++s) re[s] = im[s] = d4v{0.0, 0.0, 0.0, 0.0};
+
+    // k past m reads the last point against a zero of the matrix; rows and lines past m are not stored
+    auto load = [&](auto dir, int p, d2v (&u)[2 * KP], d2v (&f)[KP]) {
+        constexpr bool Z = decltype(dir)::value;
+        const SumProd& q = job.prod[Z][p];
+        const d2v* S = q.src + base;
+        const d2v* F = (const d2v*)q.mat + (size_t)(Z ? tz : ty) * (2 * nt) * 64 + lane;
+        const int line = min((Z ? y16 : z16) + l16, m - 1);
+#pragma unroll
+        for (int kp = 0; kp < KP; ++kp) {
+            f[kp] = F[kp * 64];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k = min(8 * kp + 4 * h + l4, m - 1);
+                u[2 * kp + h] = S[Z ? k * m + line : line * m + k];
+            }
+        }
+    };
+    auto mul = [&](auto dir, double coef, const d2v (&u)[2 * KP], const d2v (&f)[KP], d4v& r, d4v& i) {
+        constexpr bool Z = decltype(dir)::value;
+#pragma unroll
+        for (int kp = 0; kp < KP; ++kp)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const double d = coef * f[kp][h];
+                const d2v x = u[2 * kp + h];
+                r = Z ? mfma(d, x[0], r) : mfma(x[0], d, r);
+                i = Z ? mfma(d, x[1], i) : mfma(x[1], d, i);
+            }
+    };
+    auto products = [&](auto dir) {
+        constexpr bool Z = decltype(dir)::value;
+        d2v u[NPR][2 * KP], f[NPR][KP];
+        const int n0 = job.stage[0].nprod[Z], n = n0 + (job.nstage > 1 ? job.stage[1].nprod[Z] : 0);
+#pragma unroll
+        for (int p = 0; p < NPR; ++p) load(dir, p < n ? p : 0, u[p], f[p]);
+#pragma unroll
+        for (int p = 0; p < NPR; ++p) {
+            if (p >= n) continue;
+            const double coef = job.prod[Z][p].coef;
+            if (p < n0) mul(dir, coef, u[p], f[p], re[0], im[0]);
+            else mul(dir, coef, u[p], f[p], re[1], im[1]);
+        }
+    };
+    if (wave == 1) {
+        products(std::true_type{});
+#pragma unroll
+        for (int s = 0; s < kSumStages; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ex[s][e][lane] = d2v{re[s][e], im[s][e]};
+        lds_barrier();
+        return;
+    }
+    // the first wave: the pointwise terms of both stages (unused ones are loaded in vain), then its products
+    const int y = y16 + l16;
+    unsigned o[4];
+    bool ok[4];
+    d2v t[kSumStages][kSumTerms][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int z = z16 + 4 * e + l4;
+        ok[e] = y < m && z < m;
+        o[e] = ok[e] ? z * m + y : 0;
+    }
+#pragma unroll
+    for (int s = 0; s < kSumStages; ++s)
+#pragma unroll
+        for (int j = 0; j < kSumTerms; ++j) {
+            const d2v* T = (s < job.nstage && j < job.stage[s].nterm ? job.stage[s].term[j].t : job.stage[0].term[0].t) + base;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[s][j][e] = T[o[e]];
+        }
+    products(std::false_type{});
+    lds_barrier();
+    const double xa = a.alp * (double)mode;
+    d2v x[4];
+#pragma unroll
+    for (int s = 0; s < kSumStages; ++s) {
+        if (s >= job.nstage) continue;
+        const SumStage& st = job.stage[s];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const d2v p = d2v{re[s][e], im[s][e]} + ex[s][e][lane];
+            x[e] = s > 0 && st.keep != 0.0 ? st.keep * x[e] + p : p;
+        }
+#pragma unroll
+        for (int j = 0; j < kSumTerms; ++j) {
+            if (j >= st.nterm) continue;
+            const double cr = st.term[j].cr + st.term[j].crx * xa * xa, ci = st.term[j].ci * xa;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] += cr * t[s][j][e] + ci * d2v{-t[s][j][e][1], t[s][j][e][0]};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (mode == 0) x[e][0] += st.c0;
+            if (ok[e]) (st.out + base)[o[e]] = x[e];
+        }
+    }
+}
+
+// Up to the size where the unfolded products cost more than the launches saved: a step of 64^2 x 48 modes
+// (modes x tiles x fragment pairs 6144) takes 442 us against 461 of the y and z launches, 64^2 x 64 (8192)
+// 471 against 449, 33^2 x 128 (5760) 341 against 389, 17^2 x 256 (3072) 259 against 319.
+bool sums_supported(int m, int nmodes)
+{
+    const long nt = (m + 15) / 16;
+    return m <= kSumMaxM && nmodes * nt * nt * ((m + 7) / 8) <= 7168;
+}
+
+template <int KP>
+static void launch_sums_kp(const SumArgs& a, int np, dim3 grid, hipStream_t st)
+{
+    if (np <= 1) hipLaunchKernelGGL((k_sums<KP, 1>), grid, dim3(128), 0, st, a);
+    else hipLaunchKernelGGL((k_sums<KP, kSumProds>), grid, dim3(128), 0, st, a);
+}
+
+hipError_t launch_sums(const SumArgs& a, hipStream_t st)
+{
+    if (a.njobs < 0 || a.njobs > kSumJobs || a.m < kMinM || a.m > kSumMaxM) return hipErrorInvalidValue;
+    int most = 0;
+    for (int j = 0; j < a.njobs; ++j) {
+        const SumJob& J = a.job[j];
+        int np[2] = {0, 0};
+        if (J.nstage < 1 || J.nstage > kSumStages) return hipErrorInvalidValue;
+        for (int s = 0; s < J.nstage; ++s) {
+            const SumStage& S = J.stage[s];
+            if (!S.out || S.nterm < 0 || S.nterm > kSumTerms || S.nprod[0] < 0 || S.nprod[1] < 0) return hipErrorInvalidValue;
+            for (int t = 0; t < S.nterm; ++t)
+                if (!S.term[t].t) return hipErrorInvalidValue;
+            for (int d = 0; d < 2; ++d) np[d] += S.nprod[d];
+        }
+        if (J.stage[0].nterm < 1) return hipErrorInvalidValue;   // (the address that unused terms read)
+        for (int d = 0; d < 2; ++d) {
+            if (np[d] > kSumProds || !J.prod[d][0].src || !J.prod[d][0].mat) return hipErrorInvalidValue;
+            for (int p = 0; p < np[d]; ++p)
+                if (!J.prod[d][p].src || !J.prod[d][p].mat) return hipErrorInvalidValue;
+            most = std::max(most, np[d]);
+        }
+    }
+    if (a.njobs == 0 || a.nmodes <= 0) return hipSuccess;
+    const int nt = (a.m + 15) / 16;
+    const long total = (long)a.njobs * a.nmodes * nt * nt;
+    if (total >= 1L << 30) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((total + 7) / 8 * 8));
+    switch ((a.m + 7) / 8) {
+        case 1: launch_sums_kp<1>(a, most, grid, st); break;
+        case 2: launch_sums_kp<2>(a, most, grid, st); break;
+        case 3: launch_sums_kp<3>(a, most, grid, st); break;
+        case 4: launch_sums_kp<4>(a, most, grid, st); break;
+        case 5: launch_sums_kp<5>(a, most, grid, st); break;
+        case 6: launch_sums_kp<6>(a, most, grid, st); break;
+        case 7: launch_sums_kp<7>(a, most, grid, st); break;
+        default: launch_sums_kp<8>(a, most, grid, st); break;
+    }
     return hipGetLastError();
 }
 
