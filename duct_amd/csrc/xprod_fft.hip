@@ -6,9 +6,11 @@
 // What bounds it: the nine fields of M modes per line cross HBM once, 9 x 16 B x M per line, and
 // everything else happens in registers and LDS.
 //
-// Two real lines share a complex transform (u + i v of a line; w of two neighbouring lines; the
-// products as uu + i vv, ww + i uv, uw + i vw), so a line costs 1.5 inverse and 3 forward complex
-// transforms of X points.  A transform is a Stockham sequence of passes of radix 2, 3, 4, 5 or 8
+// Two neighbouring lines share a complex transform, for each of u, v, w and each product, so a line
+// costs 1.5 inverse and 3 forward complex transforms of X points.  (Sharing it between u and v of a line,
+// and between uu and vv, leaves the rounding of the larger in the smaller: at 384 x 128 x 257^2 the v and w
+// components of a duct flow's advection were 7.9e-15 and 6.4e-15 off, now 5.3e-15 and 5.4e-15; with rocFFT's
+// transforms of one real line each 5.6e-15 and 5.5e-15.)  A transform is a Stockham sequence of passes of radix 2, 3, 4, 5 or 8
 // through one LDS image per line: a workgroup reads all its butterflies into registers, waits,
 // and writes them back, so one image is enough.  The inverse's last pass and the forward's first
 // have the same radix R (4, 6 or 10): a butterfly's outputs x = j + i X/R of the one are its
@@ -21,12 +23,12 @@
 // is odd.  Consecutive workgroups of one XCD own neighbouring tiles, so the cache lines that two
 // tiles share are fetched into one L2.
 //
-// Measured (the 9 fields' bytes over the launch): 535 us at 384 points x 128 modes x 257^2 lines
-// (2.3 TB/s; rocFFT's batched transforms with pad, multiply and pack kernels, which this replaces,
-// took 5690 us), 41 us at 120 x 40 x 97^2 (257 us), 72 us at 144 x 48 x 129^2 (the dense transform
+// Measured (the 9 fields' bytes over the launch): 615 us at 384 points x 128 modes x 257^2 lines
+// (2.0 TB/s; rocFFT's batched transforms with pad, multiply and pack kernels, which this replaces,
+// took 5690 us), 44 us at 120 x 40 x 97^2 (257 us), 72 us at 144 x 48 x 129^2 (the dense transform
 // of k_xprod: 129 us).  Counters at 384 points: the vector units issue a third of the time, LDS is
 // busy a third; the rest is waits at the barriers between passes.  The roots of unity are read from
-// LDS, not from memory: gathers of 16 bytes per lane through the L1 cost 654 against 535 us.
+// LDS, not from memory: gathers of 16 bytes per lane through the L1 cost 1.2 times as much.
 #include <algorithm>
 #include <cmath>
 #include <functional>
@@ -191,11 +193,6 @@ __device__ __forceinline__ void run_pass(d2v* Z, const XfftPass& p, const d2v* t
     }
 }
 
-__device__ __forceinline__ d2v lane_xor1(d2v v)
-{
-    return d2v{__shfl_xor(v[0], 1, 64), __shfl_xor(v[1], 1, 64)};
-}
-
 }  // namespace
 
 template <int R>
@@ -212,17 +209,22 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
     const long L0 = tile * T;
     const long nlines = a.lines - L0;          // valid lines of this tile (>= 1)
 
-    constexpr int PT = xfft_per_thread(R), IT = (PT + 2) / 3;   // 3 M <= X: at most X / 3 coefficients per line
-    d2v cu[IT], cv[IT], cw[IT];
+    // a thread's coefficients: mode k of the pair of lines 2 p and 2 p + 1
+    constexpr int PT = xfft_per_thread(R), IT = (PT + 5) / 6;   // 3 M <= X: at most X / 3 coefficients per line
+    d2v cu[IT][2], cv[IT][2], cw[IT][2];
+    const int hT = T >> 1;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int e = tid + it * nth, l = e & (T - 1), k = e >> a.logT;
-        const bool ok = k < M && l < nlines;
-        const size_t idx = ok ? (size_t)k * a.lines + L0 + l : 0;
-        cu[it] = a.in[0][idx];
-        cv[it] = a.in[1][idx];
-        cw[it] = a.in[2][idx];
-        if (!ok) cu[it] = cv[it] = cw[it] = d2v{0.0, 0.0};
+        const int e = tid + it * nth, p = e & (hT - 1), k = e >> (a.logT - 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool ok = k < M && 2 * p + h < nlines;
+            const size_t idx = ok ? (size_t)k * a.lines + L0 + 2 * p + h : 0;
+            cu[it][h] = a.in[0][idx];
+            cv[it][h] = a.in[1][idx];
+            cw[it][h] = a.in[2][idx];
+            if (!ok) cu[it][h] = cv[it][h] = cw[it][h] = d2v{0.0, 0.0};
+        }
     }
     auto clear = [&](int nl) {                 // the modes that the 3/2 rule leaves empty
         const int nz = X - 2 * M + 1;
@@ -233,28 +235,32 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
     };
 
     for (int e = tid; e < X; e += nth) tw[pad8(e)] = a.tw[e];
-    // ---- u + i v of every line
+    // ---- u and v of two lines at a time: line 2 p + i line (2 p + 1)
+    auto pack = [&](d2v* z, const d2v (&c)[2], int k) {
+        const d2v x = c[0], y = c[1];
+        if (k == 0) {
+            z[0] = d2v{x[0], y[0]};   // FFTW's c2r ignores Im of mode 0
+        } else {
+            z[pad8(k)] = d2v{x[0] - y[1], x[1] + y[0]};
+            z[pad8(X - k)] = d2v{x[0] + y[1], y[0] - x[1]};
+        }
+    };
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int e = tid + it * nth, l = e & (T - 1), k = e >> a.logT;
+        const int e = tid + it * nth, p = e & (hT - 1), k = e >> (a.logT - 1);
         if (k < M) {
-            const d2v u = cu[it], v = cv[it];
-            if (k == 0) {
-                Z[l * ld] = d2v{u[0], v[0]};   // FFTW's c2r ignores Im of mode 0
-            } else {
-                Z[l * ld + pad8(k)] = d2v{u[0] - v[1], u[1] + v[0]};
-                Z[l * ld + pad8(X - k)] = d2v{u[0] + v[1], v[0] - u[1]};
-            }
+            pack(Z + 2 * p * ld, cu[it], k);
+            pack(Z + (2 * p + 1) * ld, cv[it], k);
         }
     }
     clear(T);
     lds_barrier();
     for (int i = 0; i < a.ninv; ++i) run_pass<PT, true>(Z, a.inv[i], tw, T, ld, tid, nth);
 
-    // ---- the last inverse pass: butterfly j of the lines 2 pr and 2 pr + 1
+    // ---- the last inverse pass: butterfly j of the pair of lines 2 pr and 2 pr + 1
     const bool own = tid < (T >> 1) * nf;
     const int pr = own ? div_by(tid, a.inv_nf) : 0, j = own ? tid - pr * nf : 0;
-    d2v ua[R], ub[R], ww[R];                   // (u, v) of the two lines; (w of line 2 pr, w of line 2 pr + 1)
+    d2v uu[R], vv[R], ww[R];                   // u, v, w of the pair: (line 2 pr, line 2 pr + 1)
     auto last = [&](const d2v* src, d2v (&v)[R]) {
 #pragma unroll
         for (int i = 0; i < R; ++i) v[i] = src[pad8(j + i * nf)];
@@ -263,34 +269,23 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         dft<R, true>(v);
     };
     if (own) {
-        last(Z + (2 * pr) * ld, ua);
-        last(Z + (2 * pr + 1) * ld, ub);
+        last(Z + (2 * pr) * ld, uu);
+        last(Z + (2 * pr + 1) * ld, vv);
     }
     lds_barrier();
 
-    // ---- w of two lines at a time (lane l holds line l's coefficient, its neighbour the partner's)
+    // ---- w
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        const int e = tid + it * nth, l = e & (T - 1), k = e >> a.logT;
-        const d2v other = lane_xor1(cw[it]);
-        if (k < M) {
-            const d2v x = (l & 1) ? other : cw[it], y = (l & 1) ? cw[it] : other;
-            d2v* z = Z + (l >> 1) * ld;
-            if (k == 0) {
-                if (!(l & 1)) z[0] = d2v{x[0], y[0]};
-            } else if (!(l & 1)) {
-                z[pad8(k)] = d2v{x[0] - y[1], x[1] + y[0]};
-            } else {
-                z[pad8(X - k)] = d2v{x[0] + y[1], y[0] - x[1]};
-            }
-        }
+        const int e = tid + it * nth, p = e & (hT - 1), k = e >> (a.logT - 1);
+        if (k < M) pack(Z + p * ld, cw[it], k);
     }
     clear(T >> 1);
     lds_barrier();
     for (int i = 0; i < a.ninv; ++i) run_pass<PT, true>(Z, a.inv[i], tw, T >> 1, ld, tid, nth);
     if (own) last(Z + pr * ld, ww);
 
-    // ---- the products, two per complex transform: uu + i vv, ww + i uv, uw + i vw
+    // ---- the products of the pair, one per complex transform: uu and vv, ww and uv, uw and vw
     for (int q = 0; q < 3; ++q) {
         // (opaque per round: the addresses of a round are cheap to form and would otherwise all be
         // kept in registers across the rounds)
@@ -303,8 +298,8 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
                 d2v z[R];
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
-                    const double u = h ? ub[i][0] : ua[i][0], v = h ? ub[i][1] : ua[i][1], w = ww[i][h];
-                    z[i] = q == 0 ? d2v{u * u, v * v} : q == 1 ? d2v{w * w, u * v} : d2v{u * w, v * w};
+                    const d2v f = q == 0 ? (h ? vv[i] : uu[i]) : q == 1 ? (h ? uu[i] : ww[i]) : (h ? vv[i] : uu[i]);
+                    z[i] = f * (q == 0 ? f : q == 1 ? (h ? vv[i] : ww[i]) : ww[i]);
                 }
                 dft<R, false>(z);
                 d2v* out = Z + (2 * pq + h) * ld;
@@ -314,16 +309,17 @@ __global__ __launch_bounds__(kXfftMaxThreads, R == 4 ? 3 : 2) void k_xprod_fft(X
         }
         lds_barrier();
         for (int i = 0; i < a.nfwd; ++i) run_pass<PT, false>(Z, a.fwd[i], tw, T, ld, tq, nth);
-        d2v* O0 = a.out[2 * q];
-        d2v* O1 = a.out[2 * q + 1];
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
-            const int e = tq + it * nth, l = e & (T - 1), k = e >> a.logT;
-            if (k < M && l < nlines) {
-                const d2v f = Z[l * ld + pad8(k)], g = Z[l * ld + pad8(k ? X - k : 0)];
-                const size_t idx = (size_t)k * a.lines + L0 + l;
-                O0[idx] = a.scale * d2v{f[0] + g[0], f[1] - g[1]};
-                O1[idx] = a.scale * d2v{f[1] + g[1], g[0] - f[0]};
+            const int e = tq + it * nth, p = e & (hT - 1), k = e >> (a.logT - 1);
+            if (k >= M) continue;
+            const size_t idx = (size_t)k * a.lines + L0 + 2 * p;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const d2v* z = Z + (2 * p + h) * ld;
+                const d2v f = z[pad8(k)], g = z[pad8(k ? X - k : 0)];
+                if (2 * p < nlines) a.out[2 * q + h][idx] = a.scale * d2v{f[0] + g[0], f[1] - g[1]};
+                if (2 * p + 1 < nlines) a.out[2 * q + h][idx + 1] = a.scale * d2v{f[1] + g[1], g[0] - f[0]};
             }
         }
     }
@@ -413,7 +409,7 @@ hipError_t launch_xprod_fft(const XprodArgs& x, const d2v* tw, hipStream_t st)
         return (need + 63) / 64 * 64;
     };
     // Lines per workgroup: 8 (128 bytes of a mode per access) while 256 threads hold them (more
-    // threads wait longer at each barrier: 957 against 535 us at 384 x 257^2 for 8 and 4 lines), 4
+    // threads wait longer at each barrier: 8 lines took 1.8 times as long as 4 at 384 x 257^2), 4
     // where 8 leave fewer than two workgroups per CU (16.8 against 14.0 us at 48 x 33^2).
     int T = 2, logT = 1;
     while (T < 8 && threads(T * 2) <= 256 && !(T == 4 && a.lines < 8 * 512)) { T *= 2; ++logT; }
