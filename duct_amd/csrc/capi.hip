@@ -511,10 +511,8 @@ struct PlaneLaunch {
 bool plane_fields(std::initializer_list<const FieldGroup*> groups)
 {
     std::vector<std::pair<uintptr_t, uintptr_t>> in, out;
-    long planes = 0;
-    for (const FieldGroup* g : groups) planes += 2L * g->nf * g->nmodes;
     for (const FieldGroup* g : groups) {
-        if (!plane_supported(g->m, g->m, planes)) return false;
+        if (!plane_supported(g->m, g->m)) return false;
         const uintptr_t bytes = (uintptr_t)g->nmodes * g->m * g->m * sizeof(d2v);
         for (int f = 0; f < g->nf; ++f) {
             in.emplace_back((uintptr_t)g->in[f], (uintptr_t)g->in[f] + bytes);
@@ -530,8 +528,14 @@ bool plane_fields(std::initializer_list<const FieldGroup*> groups)
     return true;
 }
 
-// Solved without the folded bases.
-bool unfolded_group(const FieldGroup& g, int bidx) { return !(L.basis[bidx].NH > 0 && L.fold > bidx); }
+// Solved without the folded bases: where folding is off, and where whole solves in LDS take less time.  The
+// folded passes pad every plane to 128 (m <= 130) and take six launches and more: 4 fields of 67^2 x 16 modes
+// 159 us against 40 in LDS, 97^2 x 256 534 against 297, 114^2 x 256 571 against 547.  Only many full planes
+// are faster folded: 129^2 x 128 350 against 329, 129^2 x 256 589 against 654.
+bool unfolded_group(const FieldGroup& g, int bidx)
+{
+    return !(L.basis[bidx].NH > 0 && L.fold > bidx) || (plane_supported(g.m, g.m) && (g.n <= 112 || g.nmodes <= 128));
+}
 
 int check_group(const FieldGroup& g, int bidx)
 {
@@ -541,9 +545,9 @@ int check_group(const FieldGroup& g, int bidx)
     return OK;
 }
 
-// lds: the unfolded solves may keep their planes in LDS (not beside another group's passes, which then
-// wait for the CUs: 742 against 715 us at 129^2 x 256 modes x 4)
-int run_group(const FieldGroup& g, int bidx, int bmode, bool lds = true)
+// lds: whole solves in LDS where the group's planes fit (false beside a group whose right-hand sides this
+// one's solutions overlap: they would be written before the other group has read them)
+int run_group(const FieldGroup& g, int bidx, int bmode, bool lds)
 {
     int st0 = check_group(g, bidx);
     if (st0) return st0;
@@ -551,7 +555,7 @@ int run_group(const FieldGroup& g, int bidx, int bmode, bool lds = true)
     // folded, except the low Poisson modes of a Neumann group (kLowXlam)
     const int klow = bidx == 1 ? low_mode_prefix(g) : 0;
     int st;
-    if (klow > 0 && (st = run_group_unfolded(mode_range(g, 0, klow), bidx, bmode))) return st;
+    if (klow > 0 && (st = run_group_unfolded(mode_range(g, 0, klow), bidx, bmode, lds))) return st;
     if (klow < g.nmodes) return run_group_fold(mode_range(g, klow, g.nmodes - klow), bidx, bmode);
     return OK;
 }
@@ -1125,7 +1129,8 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
         }
     }
     // Planes that fit LDS: every field of both boundary types in one launch.
-    if ((!g[0].nf || unfolded_group(g[0], 0)) && (!g[1].nf || unfolded_group(g[1], 1)) && plane_fields({&g[0], &g[1]})) {
+    const bool lds = plane_fields({&g[0], &g[1]});
+    if (lds && (!g[0].nf || unfolded_group(g[0], 0)) && (!g[1].nf || unfolded_group(g[1], 1))) {
         PlaneLaunch p(g[0], dir_bmode);
         for (int bidx = 0; bidx < 2; ++bidx) {
             if (!g[bidx].nf) continue;
@@ -1145,11 +1150,11 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
         }
         HIPCHK(hipEventRecord(L.ev_fork, L.stream));
         HIPCHK(hipStreamWaitEvent(L.side, L.ev_fork, 0));
-        st = run_group(g[0], 0, dir_bmode, false);
+        st = run_group(g[0], 0, dir_bmode, lds);
         int st_side;
         {
             SideLane lane;
-            st_side = run_group(g[1], 1, dir_bmode, false);
+            st_side = run_group(g[1], 1, dir_bmode, lds);
         }
         HIPCHK(hipEventRecord(L.ev_join, L.side));
         HIPCHK(hipStreamWaitEvent(L.stream, L.ev_join, 0));
@@ -1157,7 +1162,7 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
     }
     for (int bidx = 0; bidx < 2; ++bidx) {
         if (g[bidx].nf == 0) continue;
-        st = run_group(g[bidx], bidx, dir_bmode, !(g[0].nf && g[1].nf));
+        st = run_group(g[bidx], bidx, dir_bmode, lds);
         if (st) return st;
     }
     return OK;
@@ -1938,7 +1943,7 @@ static int solve_plane(const char* bound, double xlambda, int imode)
         bc.D2b = B.D2b;
         HIPCHK(launch_bc_correct(bc, L.stream));
     }
-    return run_group(g, bidx, BND_DIR_KEEP);
+    return run_group(g, bidx, BND_DIR_KEEP, true);
 }
 
 static int plane_buffers(int m)
@@ -2592,7 +2597,7 @@ int duct_helm3d_temp_dev_(const duct_devptr_t* rhs, const duct_devptr_t* sol, co
     if (!T.ready || T.my != *my || T.mz != *mz)
         return fail(ERR_NOT_SETUP, "duct_setup_temp_ not called for my=%d, mz=%d", *my, *mz);
     const int NP = T.NP, ny = *my - 2, nz = *mz - 2, M = *nmodes;
-    if (plane_supported(*my, *mz, 2L * M)) {
+    if (plane_supported(*my, *mz)) {
         PlaneArgs pa{};
         pa.in[0] = (const d2v*)*rhs;
         pa.out[0] = (d2v*)*sol;

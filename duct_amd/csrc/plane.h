@@ -41,8 +41,8 @@ struct PlaneArgs {
     const double* vec;
     int by1, by2, bz1, bz2;
 };
-// whether planes of these sizes are solved in LDS, `planes` real ones in a call
-bool plane_supported(int my, int mz, long planes);
+// whether planes of these sizes fit LDS
+bool plane_supported(int my, int mz);
 hipError_t launch_plane(int kind, const PlaneArgs& a, hipStream_t st);
 
 }  // namespace duct

@@ -18,11 +18,12 @@
 // Re and Im of a plane are neighbouring workgroups of one XCD: each reads and writes its half of
 // the same cache lines.  Workgroups are as many as the CUs hold and walk their planes.
 //
-// What bounds it: the FP64 matrix cores.  At RT = 8 a plane takes ~167e3 cycles of which its MFMAs are
+// What bounds it: the FP64 matrix cores.  At RT = 8 a plane takes ~155e3 cycles of which its MFMAs are
 // 131e3; the rest is what one workgroup per CU cannot overlap: the writes between the passes (~4e3
-// each), the divide (~9e3), the stores and walls (~10e3).  u, v, w and p at 129^2 x 64 modes take 186 us
-// (8 launches and 216 us before), one field of 33^2 x 16 11 us (31), 65^2 x 128 x 4 57 us (139), the
-// mixed walls at 97 x 129 x 64 81 us (140).
+// each), the divide (~9e3), the stores and walls.  u, v, w and p at 129^2 x 64 modes take 170 us
+// (8 launches and 216 us as passes over planar intermediates), at 129^2 x 256 652 us (736), one field of
+// 33^2 x 16 11 us (31), 97^2 x 40 51 us for the Neumann field, the mixed walls at 97 x 129 x 64 81 us (140)
+// and at 129 x 129 x 400 362 us (483).
 #include <algorithm>
 
 #include "plane.h"
@@ -51,10 +52,10 @@ __device__ __forceinline__ double line_sum(double v)
 }
 
 // waves per SIMD that the LDS admits
-constexpr int plane_waves(int RT, int NW)
+constexpr int plane_waves(int RT, int NW, int kind)
 {
-    const int lds = (16 * RT * (16 * RT + 1) + 6 * 16 * RT + 64) * 8, wgs = 163840 / lds;
-    const int waves = (wgs < 1 ? 1 : wgs) * NW / 4;
+    const int lds = (16 * RT * (16 * RT + 1) + (kind == PLANE_FWD ? 4 : 6) * 16 * RT + 4 * NW) * 8, wgs = (int)kLdsPerCu / lds;
+    const int waves = ((wgs < 1 ? 1 : wgs) * NW + 3) / 4;
     return waves < 2 ? 2 : waves > 4 ? 4 : waves;
 }
 
@@ -86,7 +87,7 @@ __device__ __forceinline__ void wall_line(int t1, int t2, const WallRows& w, dou
 }  // namespace
 
 template <int RT, int RR, int CC, int KIND>
-__global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / RR) * (RT / CC))) void k_plane(PlaneArgs a)
+__global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / RR) * (RT / CC), KIND)) void k_plane(PlaneArgs a)
 {
     constexpr int N = 16 * RT, LD = N + 1, WC = RT / CC, NW = (RT / RR) * WC, NTH = 64 * NW;
     // One workgroup fills the LDS (RT 7 and 8): its next plane is loaded under the last pass.  All CUs
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / R
     double* X = sm;              // [column][row], stride LD
     double* lam = X + N * LD;    // eigenvalues of the two bases (WALL: along y and along z)
     double* red = lam + 2 * N;   // 4 NW: the waves' partial sums
-    double* vec = red + 4 * NW;  // ADJ, WALL: 4 N, the vectors of the wall terms
+    double* vec = red + 4 * NW;  // ADJ, WALL: 4 N, the vectors of the wall terms; FWD, WALL: rows 1 and m of D
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -143,6 +144,9 @@ __global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / R
         const double* src = KIND == PLANE_WALL ? (t < N ? a.b[0].lamy : a.b[0].lamz) : a.b[t / N].lamy;
         lam[t] = src ? src[t % N] : 0.0;
     }
+    if (KIND == PLANE_FWD && a.b[1].DC)
+        for (int t = tid; t < 2 * N; t += NTH)
+            vec[t] = t % N < ny ? a.b[1].DC[(t < N ? 0 : my - 1) + (size_t)(t % N + 1) * my] : 0.0;
 
     double v[NV];
     auto load = [&](const double* in, int it) {
@@ -453,25 +457,27 @@ __global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / R
     }
 
     // ---- edges of the Neumann field (solvediag.f90:251-322) and of the walls (solvediag_temp.f90): the
-    // sums along y and z with the derivative rows, four threads per line
+    // sums along y and z with the derivative rows, several threads per line
+    if (KIND == PLANE_WALL)
+        for (int t = tid; t < 4 * N; t += NTH) {   // (the wall vectors of the right-hand side are used up)
+            const int i = t % N, d = t / N;
+            vec[t] = i < (d < 2 ? ny : nz) ? (d < 2 ? Dy0 + d * my : Dz0 + (d - 2) * mz)[i + 1] : 0.0;
+        }
     put();
-    const bool nn = KIND == PLANE_FWD;
-    const double* D0y = nn ? B.DC : Dy0;                    // row 1 of D along y, entries Dsy apart
-    const double* Dmy = nn ? B.DC + (my - 1) : Dy0 + my;
-    const double* D0z = nn ? B.DC : Dz0;
-    const double* Dmz = nn ? B.DC + (mz - 1) : Dz0 + mz;
-    const int ds = nn ? my : 1;
     // LPL lanes per line: line z = c over y, line y = c over z (threads past the last line repeat it)
     const int c = min(tid / LPL, N - 1), q = tid % LPL;
     const bool line = tid / LPL < N;
     double s0y = 0.0, smy = 0.0, s0z = 0.0, smz = 0.0;
-    for (int t = q; t < N; t += LPL) {
-        const double uy = X[c * LD + t], uz = X[t * LD + c];
-        const int ty = t < ny ? t + 1 : 0, tz = t < nz ? t + 1 : 0;   // (the padding of X is zero)
-        s0y += D0y[(size_t)ty * ds] * uy;
-        smy += Dmy[(size_t)ty * ds] * uy;
-        s0z += D0z[(size_t)tz * ds] * uz;
-        smz += Dmz[(size_t)tz * ds] * uz;
+    // each sum ends with its largest terms, at its own wall: the other way round the small ones would be
+    // rounded to the large ones' last place, and phi's walls are what grad(phi) multiplies by m^2 / 3
+    const double* vz = KIND == PLANE_WALL ? vec + 2 * N : vec;
+#pragma unroll 4
+    for (int i = 0; i < N / LPL; ++i) {
+        const int t = q + i * LPL, r = N - LPL + q - i * LPL;
+        s0y += vec[r] * X[c * LD + r];
+        smy += vec[N + t] * X[c * LD + t];
+        s0z += vz[r] * X[r * LD + c];
+        smz += vz[N + t] * X[t * LD + c];
     }
     s0y = line_sum<LPL>(s0y);
     smy = line_sum<LPL>(smy);
@@ -549,20 +555,16 @@ __global__ __launch_bounds__(64 * (RT / RR) * (RT / CC), plane_waves(RT, (RT / R
     }
 }
 
-bool plane_supported(int my, int mz, long planes)
+bool plane_supported(int my, int mz)
 {
-    if (my < kMinM || mz < kMinM || my - 2 > kPlaneMaxN || mz - 2 > kPlaneMaxN) return false;
-    // At eight tiles the planes fill the padding of the projection passes too, and these, two workgroups
-    // to a CU, reach more of the matrix cores once there are many planes: 715 against 782 us for 2047
-    // planes of 129^2 (197 against 210 us, edges and gauge included, for 508).
-    return std::max(my, mz) - 2 <= 112 || planes <= 640;
+    return my >= kMinM && mz >= kMinM && my - 2 <= kPlaneMaxN && mz - 2 <= kPlaneMaxN;
 }
 
 template <int RT, int RR, int CC>
 static hipError_t launch_plane_rt(int kind, const PlaneArgs& a, hipStream_t st)
 {
     constexpr int N = 16 * RT, NW = (RT / RR) * (RT / CC);
-    const size_t lds = ((size_t)N * (N + 1) + (kind == PLANE_FWD ? 2 : 6) * N + 4 * NW) * sizeof(double);
+    const size_t lds = ((size_t)N * (N + 1) + (kind == PLANE_FWD ? 4 : 6) * N + 4 * NW) * sizeof(double);
     // as many workgroups as fit the CUs' LDS at once (and 16 waves of each), a multiple of the XCDs
     int dev = 0, ncu = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -581,7 +583,7 @@ static hipError_t launch_plane_rt(int kind, const PlaneArgs& a, hipStream_t st)
 
 hipError_t launch_plane(int kind, const PlaneArgs& a, hipStream_t st)
 {
-    if (!plane_supported(a.my, a.mz, 0) || a.nf < 0 || a.nf > kMaxFields) return hipErrorInvalidValue;
+    if (!plane_supported(a.my, a.mz) || a.nf < 0 || a.nf > kMaxFields) return hipErrorInvalidValue;
     if (a.nf == 0 || a.nmodes <= 0) return hipSuccess;
     const int n = (a.my > a.mz ? a.my : a.mz) - 2;
     switch ((n + 15) / 16) {

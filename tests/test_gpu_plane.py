@@ -107,3 +107,37 @@ def test_plane_walls_match_oracle(dev, my, mz, walls):
     e = relerr(sol.cpu().numpy(), ref)
     print("my=%d mz=%d %s rel.err %.2e" % (my, mz, walls, e), flush=True)
     assert e <= TOL
+
+
+def test_plane_many_planes_and_folding(dev):
+    """More planes than the CUs hold at once, against the projection passes; and the folded solver where it
+    leaves whole solves to LDS: the same bits with folding on as off."""
+    import torch
+    from duct_amd import solver
+    m, M = 129, 165
+    dev.setup(m)
+    f = [field(M, m, k) for k in range(2)]
+    for bounds in ("dd", "nn"):
+        sol = [torch.full((M, m, m), float("nan"), dtype=torch.complex128, device="cuda") for _ in f]
+        dev.helm3d_batch([torch.from_numpy(x).cuda() for x in f], sol, bounds, [700.0, 3.0], alp=0.9, ib=2)
+        a, b = (torch.from_numpy(x).cuda() for x in f)
+        dev.helm3d_batch([a, b], [b, a], bounds, [700.0, 3.0], alp=0.9, ib=2)
+        torch.cuda.synchronize()
+        for s, r in zip(sol, (b, a)):
+            e = relerr(s.cpu().numpy(), r.cpu().numpy())
+            print("m=%d M=%d %s rel.err %.2e" % (m, M, bounds, e), flush=True)
+            assert e <= TOL
+    for m, M in ((67, 4), (114, 3), (129, 4)):
+        dev.setup(m)
+        f = [field(M, m, 7 * m + k) for k in range(2)]
+        got = []
+        for fold in (0, 2):
+            solver.set_fold(fold)
+            try:
+                s = [torch.full((M, m, m), float("nan"), dtype=torch.complex128, device="cuda") for _ in f]
+                dev.helm3d_batch([torch.from_numpy(x).cuda() for x in f], s, "dn", [700.0, 0.0], alp=0.9)
+                torch.cuda.synchronize()
+                got.append([x.cpu().numpy() for x in s])
+            finally:
+                solver.set_fold(0)
+        assert all(np.array_equal(x, y) for x, y in zip(*got))
