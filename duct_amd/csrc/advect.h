@@ -68,12 +68,10 @@ struct DerivyzArgs {
 hipError_t launch_derivyz(const DerivyzArgs& a, hipStream_t st);
 // Chebyshev transform matrices (column-major m x m): fwd = phys -> coefficients, inv = the inverse.
 void build_cheb_transforms(int m, std::vector<double>& fwd, std::vector<double>& inv);
-// The rows y < ceil(m/2) of D (fold1), D2 (fold2) and D^T (fold1t) with the contraction folded about
-// the centre node: [Dp | Dm] in fragment layout, each (16 ceil(ceil(m/2)/16))^2, then the centre row
-// (the derivative products of k_lines on the even and odd parts of their input).
-void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2, std::vector<double>& fold1t);
-// D and D2 themselves, column-major (k_sums)
-void build_colloc_full(int m, std::vector<double>& full1, std::vector<double>& full2);
+// fold: the rows y < ceil(m/2) of D and D2 with the contraction folded about the centre node: [Dp | Dm] in
+// fragment layout, each (16 ceil(ceil(m/2)/16))^2, then the centre row (the derivative products of k_lines on
+// the even and odd parts of their input).  full: D, D2 and D^T themselves, column-major (k_line, k_sums).
+void build_colloc(int m, std::vector<double> (&fold)[2], std::vector<double> (&full)[3]);
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd);
 
 // Sizes beyond the dense x-DFT kernels: batched rocFFT real transforms (capi.hip) between these

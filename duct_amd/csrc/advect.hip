@@ -380,7 +380,7 @@ void colloc_ld(int m, std::vector<long double>& D, std::vector<long double>& D2)
 namespace {
 void fold_rows(int m, const std::vector<long double>& A, bool odd, std::vector<double>& frag)
 {
-    // Rows y < he of A (D, D^T: J A J = -A, odd; D2: J A J = A) with the contraction folded about the centre:
+    // Rows y < he of A (D: J A J = -A, odd; D2: J A J = A) with the contraction folded about the centre:
     //   Dp(y, k) = A(y, k) + A(y, m-1-k)  (k < ho),  Dp(y, c) = A(y, c)  (odd m, c = ho)
     //   Dm(y, k) = A(y, k) - A(y, m-1-k)  (k < ho)
     // each sum formed in extended precision and rounded once; zero-padded to KH rows and columns, in the
@@ -407,24 +407,17 @@ void fold_rows(int m, const std::vector<long double>& A, bool odd, std::vector<d
 }
 }  // namespace
 
-void build_colloc_folded(int m, std::vector<double>& fold1, std::vector<double>& fold2, std::vector<double>& fold1t)
+void build_colloc(int m, std::vector<double> (&fold)[2], std::vector<double> (&full)[3])
 {
     std::vector<long double> D, D2;
     colloc_ld(m, D, D2);
-    fold_rows(m, D, true, fold1);
-    fold_rows(m, D2, false, fold2);
-    std::vector<long double> T((size_t)m * m);
+    fold_rows(m, D, true, fold[0]);
+    fold_rows(m, D2, false, fold[1]);
+    full[0].assign(D.begin(), D.end());
+    full[1].assign(D2.begin(), D2.end());
+    full[2].resize((size_t)m * m);
     for (int j = 0; j < m; ++j)
-        for (int i = 0; i < m; ++i) T[i + (size_t)j * m] = D[j + (size_t)i * m];
-    fold_rows(m, T, true, fold1t);
-}
-
-void build_colloc_full(int m, std::vector<double>& full1, std::vector<double>& full2)
-{
-    std::vector<long double> D, D2;
-    colloc_ld(m, D, D2);
-    full1.assign(D.begin(), D.end());
-    full2.assign(D2.begin(), D2.end());
+        for (int i = 0; i < m; ++i) full[2][i + (size_t)j * m] = full[0][j + (size_t)i * m];
 }
 
 void build_xdft(int M, int X, std::vector<double>& einv, std::vector<double>& fwd)

@@ -126,8 +126,8 @@ struct Lib {
     size_t rfield_bytes = 0;
     unsigned long long* stats = nullptr;  // residual maxima of the mixed solve
     double* tfrag[2] = {nullptr, nullptr};  // Chebyshev transforms phys->cheb, cheb->phys (transyz)
-    double* dfold[3] = {nullptr, nullptr, nullptr};  // D, D2, D^T with the contraction folded (build_colloc_folded)
-    double* dfull[2] = {nullptr, nullptr};  // D, D2 in fragments, for m <= kSumMaxM (build_colloc_full)
+    double* dfold[2] = {nullptr, nullptr};  // D, D2 with the contraction folded (build_colloc)
+    double* dfull[3] = {nullptr, nullptr, nullptr};  // D, D2, D^T as they are, in fragments (build_colloc)
     d2v* rk = nullptr;                    // Runge-Kutta substep work fields: h1..h3, advnew1..3, phi
     size_t rk_bytes = 0;
     ShenDev shen[2];                      // Shen-Legendre solve, 'd' and 'n'
@@ -1649,20 +1649,16 @@ int duct_setup_(const char* bound, const int* m_, const double* P, const double*
         if ((st = up(L.tfrag[0], f.data(), f.size()))) return st;
         build_frag(ti.data(), m, m, MP, f.data());
         if ((st = up(L.tfrag[1], f.data(), f.size()))) return st;
-        {   // D, D2 and D^T for the products in half the work (k_lines)
-            std::vector<double> f[3];
-            build_colloc_folded(m, f[0], f[1], f[2]);
-            for (int i = 0; i < 3; ++i) {
-                free_ptr(L.dfold[i]);
-                if ((st = up(L.dfold[i], f[i].data(), f[i].size()))) return st;
-            }
-        }
-        for (auto& d : L.dfull) free_ptr(d);
-        if (m <= kSumMaxM) {   // D and D2 as they are (k_sums)
-            std::vector<double> d[2];
-            build_colloc_full(m, d[0], d[1]);
+        {   // D and D2 for the products in half the work (k_lines); D, D2 and D^T as they are (k_line, k_sums)
+            std::vector<double> fold[2], full[3];
+            build_colloc(m, fold, full);
             for (int i = 0; i < 2; ++i) {
-                build_frag(d[i].data(), m, m, MP, f.data());
+                free_ptr(L.dfold[i]);
+                if ((st = up(L.dfold[i], fold[i].data(), fold[i].size()))) return st;
+            }
+            for (int i = 0; i < 3; ++i) {
+                free_ptr(L.dfull[i]);
+                build_frag(full[i].data(), m, m, MP, f.data());
                 if ((st = up(L.dfull[i], f.data(), f.size()))) return st;
             }
         }
@@ -2310,14 +2306,10 @@ int duct_colloc_deriv_dev_(const duct_devptr_t* in, const duct_devptr_t* out, co
     if ((st = check_common(*m, *nmodes))) return st;
     if (!L.dfold[0] || L.dc_m != *m)
         return fail(ERR_NOT_SETUP, "no collocation matrix for m=%d (duct_setup_ builds it)", *m);
-    LineJob j{};
-    int np = 0;
-    add_stage(j, np, {{(const d2v*)*in, L.dfold[*trans ? 2 : 0], *scal, 1}}, (d2v*)*out, {});
-    if (*beta != 0.0) {
-        j.stage[0].nterm = 1;
-        j.stage[0].term[0] = LineTerm{(const d2v*)*out, *beta, 0.0, 0.0};
-    }
-    return lines_run(*m, *nmodes, 0.0, *cdir == 'z', &j, 1);
+    LineOneArgs a{(const d2v*)*in, (d2v*)*out, L.dfull[*trans ? 2 : 0], *scal, *beta, *m, *nmodes, *cdir == 'z'};
+    Timed t(PK_DERIV);
+    HIPCHK(launch_line(a, L.stream));
+    return OK;
 }
 
 int duct_derivx_dev_(const duct_devptr_t* in, const duct_devptr_t* out, const int* m, const int* nmodes,

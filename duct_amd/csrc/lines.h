@@ -10,8 +10,8 @@ constexpr int kLineTerms = 2;    // pointwise terms of an output
 constexpr int kLineJobs = 6;     // jobs of a launch
 constexpr int kLineMaxM = 288;   // 9 row tiles of 16 folded rows
 
-// coef * A u along the launch's direction; mat: A folded (build_colloc_folded); odd: J A J = -A (the
-// first derivative and its transpose), else J A J = A (the second).
+// coef * A u along the launch's direction; mat: A folded (build_colloc); odd: J A J = -A (the
+// first derivative), else J A J = A (the second).
 struct LineProd {
     const d2v* src;
     const double* mat;
@@ -48,6 +48,16 @@ struct LinesArgs {
 };
 hipError_t launch_lines(const LinesArgs& a, hipStream_t st);
 
+// out = coef * A src + beta * out along y or z; mat: A in fragments of 16 rows (build_frag); m <= kLineMaxM
+struct LineOneArgs {
+    const d2v* src;
+    d2v* out;
+    const double* mat;
+    double coef, beta;
+    int m, nmodes, dirz;
+};
+hipError_t launch_line(const LineOneArgs& a, hipStream_t st);
+
 // The same sums along both directions in one launch, for small planes (k_sums).
 constexpr int kSumProds = 3;     // products of a job per direction
 constexpr int kSumTerms = 3;     // pointwise terms of an output
@@ -55,7 +65,7 @@ constexpr int kSumStages = 2;    // outputs of a job
 constexpr int kSumJobs = 3;      // jobs of a launch
 constexpr int kSumMaxM = 64;
 
-// coef * A u along the list's direction; mat: A in fragments of 16 rows (build_frag of build_colloc_full)
+// coef * A u along the list's direction; mat: A in fragments of 16 rows (build_frag of build_colloc)
 struct SumProd {
     const d2v* src;
     const double* mat;

@@ -355,6 +355,161 @@ hipError_t launch_lines(const LinesArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
+// ---- one product, unfolded -------------------------------------------------------------------
+// out = coef A u + beta out.  Folding halves the products but rounds each half of the rows at the scale of
+// both: through D and D^T, whose large entries stand at the walls, the gradients of the projection step came
+// out 1.6 times as far off (5.8e-15 against 3.6e-15 at 129^2 x 64), and one product per read is bound by
+// memory or nearly so.  A workgroup owns 16 lines; a wave the row tiles w and w + W, re and im: four
+// accumulators.  A last row past a multiple of 16 (m = 33, 65, 129, 257) is a dot product per line on the vector
+// units: as a tile of its own 27 us per call at 129^2 x 64 instead of 23 (folded 19).
+constexpr int kOneIT = 9;        // points per thread at most: 16 m over 64 ceil(tiles / 2) threads
+
+template <bool DIRZ>
+__global__ __launch_bounds__(576, 4) void k_line(LineOneArgs a, int nslab)
+{
+    extern __shared__ __attribute__((aligned(16))) double slab[];   // [re, im][line][k]
+    const int m = a.m, mt = (m + 15) / 16, KP = (m + 7) / 8;        // the matrix's row tiles, pairs of 4 k
+    const bool dot = m % 16 == 1;
+    const int nt = dot ? mt - 1 : mt, W = (nt + 1) / 2;             // row tiles computed as such
+    const int LDK = 8 * KP + 1, SL = 16 * LDK;
+    double* red = slab + 2 * SL;                                    // [wave][line][re, im] of the last row
+    const int nth = blockDim.x, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, l4 = lane >> 4;
+    const int per = (nslab + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);   // runs of slabs per XCD
+    if ((int)(blockIdx.x >> 3) >= per || id >= nslab) return;
+    const int L0 = id * 16, nlines = min(16, a.nmodes * m - L0);
+
+    // element offsets of a line's first point and between its points, as in k_lines
+    const size_t mm = (size_t)m * m;
+    const int mode_first = L0 / m, lrel0 = L0 - mode_first * m;
+    const size_t base0 = (size_t)mode_first * mm;
+    const float invm = 1.0f / (float)m;
+    auto line_off = [&](int l) -> unsigned {
+        const int r = lrel0 + l;
+        if constexpr (!DIRZ) return (unsigned)r * m;
+        const int dm = (int)(((float)r + 0.5f) * invm);
+        return (unsigned)dm * (unsigned)mm + (r - dm * m);
+    };
+    const unsigned sk = DIRZ ? m : 1;
+
+    const int t0 = wave, t1 = min(wave + W, nt - 1);   // the second tile of the last wave of odd nt is not stored
+    const d2v* F0 = (const d2v*)a.mat + (size_t)t0 * (2 * mt) * 64 + lane;
+    const d2v* F1 = (const d2v*)a.mat + (size_t)t1 * (2 * mt) * 64 + lane;
+    d2v f0 = F0[0], f1 = F1[0];
+    const d2v* U = a.src + base0;
+    d2v v[kOneIT];
+#pragma unroll
+    for (int it = 0; it < kOneIT; ++it) {              // points past the end read line 0's first and are not staged
+        const int e = tid + it * nth, q = (int)(((float)e + 0.5f) * invm);   // e < 16 * 288 + 576
+        int l = DIRZ ? e & 15 : q, k = DIRZ ? e >> 4 : e - q * m;
+        if (e >= 16 * m || l >= nlines) l = k = 0;
+        v[it] = U[line_off(l) + k * sk];
+    }
+#pragma unroll
+    for (int it = 0; it < kOneIT; ++it) {
+        const int e = tid + it * nth, q = (int)(((float)e + 0.5f) * invm);
+        const int l = DIRZ ? e & 15 : q, k = DIRZ ? e >> 4 : e - q * m;
+        if (e >= 16 * m) continue;
+        slab[l * LDK + k] = l < nlines ? v[it][0] : 0.0;
+        slab[SL + l * LDK + k] = l < nlines ? v[it][1] : 0.0;
+    }
+    for (int e = tid; e < 32 * (8 * KP - m); e += nth) {   // k past m, against zeros of the matrix
+        const int row = e & 31, k = m + (e >> 5);
+        slab[(row >> 4) * SL + (row & 15) * LDK + k] = 0.0;
+    }
+    lds_barrier();
+
+    d4v re0 = {0.0, 0.0, 0.0, 0.0}, im0 = re0, re1 = re0, im1 = re0;
+    const double* S0 = slab + l16 * LDK + l4;
+    auto pair = [&](int kp, const d2v& c0, const d2v& c1, d2v& n0, d2v& n1) {
+        const int kn = kp + 1 < KP ? kp + 1 : kp;
+        n0 = F0[(size_t)kn * 64];
+        n1 = F1[(size_t)kn * 64];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const double re = S0[(2 * kp + h) * 4], im = S0[SL + (2 * kp + h) * 4];
+            if constexpr (!DIRZ) {
+                re0 = mfma(re, c0[h], re0);
+                im0 = mfma(im, c0[h], im0);
+                re1 = mfma(re, c1[h], re1);
+                im1 = mfma(im, c1[h], im1);
+            } else {
+                re0 = mfma(c0[h], re, re0);
+                im0 = mfma(c0[h], im, im0);
+                re1 = mfma(c1[h], re, re1);
+                im1 = mfma(c1[h], im, im1);
+            }
+        }
+    };
+    d2v g0, g1;
+    int kp = 0;
+    for (; kp + 1 < KP; kp += 2) {
+        pair(kp, f0, f1, g0, g1);
+        pair(kp + 1, g0, g1, f0, f1);
+    }
+    if (kp < KP) pair(kp, f0, f1, g0, g1);
+
+    d2v* O = a.out + base0;
+    if (dot) {
+        const double* R = a.mat + (size_t)(mt - 1) * (2 * mt) * 128;   // A(m - 1, k): row 0 of the last tile
+        d2v c = {0.0, 0.0};
+        for (int k = tid >> 4; k < m; k += nth >> 4) {
+            const double w = R[((k >> 3) * 64 + (k & 3) * 16) * 2 + ((k >> 2) & 1)];
+            c += w * d2v{slab[l16 * LDK + k], slab[SL + l16 * LDK + k]};
+        }
+        c += d2v{__shfl_xor(c[0], 16, 64), __shfl_xor(c[1], 16, 64)};
+        c += d2v{__shfl_xor(c[0], 32, 64), __shfl_xor(c[1], 32, 64)};
+        if (l4 == 0) {
+            red[(wave * 16 + l16) * 2] = c[0];
+            red[(wave * 16 + l16) * 2 + 1] = c[1];
+        }
+        lds_barrier();
+        if (tid < nlines) {
+            c = d2v{0.0, 0.0};
+            for (int w = 0; w < W; ++w) c += d2v{red[(w * 16 + tid) * 2], red[(w * 16 + tid) * 2 + 1]};
+            const unsigned o = line_off(tid) + (m - 1) * sk;
+            c *= a.coef;
+            if (a.beta != 0.0) c += a.beta * O[o];
+            O[o] = c;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int tile = h ? wave + W : wave;
+        unsigned o[4];
+        bool ok[4];
+        d2v y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int i = 4 * e + l4, r = 16 * tile + (DIRZ ? i : l16), l = DIRZ ? l16 : i;
+            ok[e] = r < m && tile < nt && l < nlines;
+            o[e] = ok[e] ? line_off(l) + r * sk : 0;
+            y[e] = d2v{0.0, 0.0};
+        }
+        if (a.beta != 0.0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = a.beta * O[o[e]];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (ok[e]) O[o[e]] = a.coef * (h ? d2v{re1[e], im1[e]} : d2v{re0[e], im0[e]}) + y[e];
+    }
+}
+
+hipError_t launch_line(const LineOneArgs& a, hipStream_t st)
+{
+    if (!a.src || !a.out || !a.mat || a.m < kMinM || a.m > kLineMaxM) return hipErrorInvalidValue;
+    if (a.nmodes <= 0) return hipSuccess;
+    const int nslab = (int)(((long)a.nmodes * a.m + 15) / 16);
+    const int tiles = a.m % 16 == 1 ? a.m / 16 : (a.m + 15) / 16, waves = (tiles + 1) / 2;
+    const size_t lds = ((size_t)2 * 16 * (8 * ((a.m + 7) / 8) + 1) + (size_t)waves * 32) * sizeof(double);
+    const dim3 grid((unsigned)((nslab + 7) / 8 * 8)), block(64 * waves);
+    if (a.dirz) hipLaunchKernelGGL(k_line<true>, grid, block, lds, st, a, nslab);
+    else hipLaunchKernelGGL(k_line<false>, grid, block, lds, st, a, nslab);
+    return hipGetLastError();
+}
+
 // ---- small planes: both directions in one launch ----------------------------------------------
 // A small grid's step is a chain of launches that are latency: arguments, loads, a few products, stores.  Here
 // a workgroup owns one 16 x 16 tile of a job's outputs on one mode, its first wave the products along y, its

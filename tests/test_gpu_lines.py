@@ -1,10 +1,11 @@
-"""GPU tests of the folded derivative products (k_lines, through duct_colloc_deriv_dev_) at the edges
-of its tiles: one to nine row tiles, rows and contractions with remainders, odd sizes with their
-centre row, slabs of lines that span planes and end ragged, D and D^T, accumulation.
+"""GPU tests of the derivative products at the edges of their tiles: single ones (k_line, through
+duct_colloc_deriv_dev_) and the folded sums of them (k_lines, through the advection term): one to nine
+row tiles of folded rows, rows and contractions with remainders, odd sizes with their centre row, slabs
+of lines that span planes and end ragged, D and D^T, accumulation.
 
-Reference: the collocation matrix in extended precision, rounded once, times the field in float64.
-Bar: a dot product of m terms rounds to at most ~m/2 eps of the sum of the terms' magnitudes, in
-practice a few eps of it: 16 eps of max(|D| |u|).
+References: the collocation matrix in extended precision, rounded once, times the field in float64; the
+oracle's advection.  Bars: a dot product of m terms rounds to at most ~m/2 eps of the sum of the terms'
+magnitudes, in practice a few eps of it: 16 eps of max(|D| |u|); 1e-12 for the advection.
 """
 import numpy as np
 import pytest
@@ -59,3 +60,25 @@ def test_colloc_deriv_tiles(dev, m, M, trans, beta):
         e = float(np.max(np.abs(got.cpu().numpy() - ref)))
         print("m=%d M=%d %s trans=%d err %.2e bar %.2e" % (m, M, cdir, trans, e, bar), flush=True)
         assert e <= bar
+
+
+@pytest.mark.parametrize("m,M,aspect", [(65, 5, 1.0), (66, 3, 1.4), (96, 5, 1.0), (97, 3, 1.0), (130, 3, 0.8), (161, 2, 1.0),
+                                        (193, 2, 1.0), (226, 2, 1.0), (258, 1, 1.2), (287, 1, 1.0)])
+def test_folded_sums_through_advection(dev, m, M, aspect):
+    import torch
+    from duct_amd import step
+    from oracle import spectral
+    dev.setup(m)
+    rng = np.random.default_rng(100 * m + M)
+    f = []
+    for _ in range(3):
+        x = rng.standard_normal((M, m, m)) + 1j * rng.standard_normal((M, m, m))
+        x[0] = x[0].real
+        f.append(x)
+    adv = [torch.full((M, m, m), float("nan"), dtype=torch.complex128, device="cuda") for _ in range(3)]
+    step.advection(*[torch.from_numpy(x).cuda() for x in f], *adv, mgalx=4 * M, alp=0.7, aspect=aspect)
+    torch.cuda.synchronize()
+    ref = spectral.advection3d(*f, mgalx=4 * M, alp=0.7, aspect=aspect)
+    errs = [float(np.max(np.abs(a.cpu().numpy() - r)) / np.max(np.abs(r))) for a, r in zip(adv, ref)]
+    print("m=%d M=%d rel.err %s" % (m, M, errs), flush=True)
+    assert max(errs) <= 1e-12
