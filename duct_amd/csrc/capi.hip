@@ -528,13 +528,27 @@ bool plane_fields(std::initializer_list<const FieldGroup*> groups)
     return true;
 }
 
-// Solved without the folded bases: where folding is off, and where whole solves in LDS take less time.  The
-// folded passes pad every plane to 128 (m <= 130) and take six launches and more: 4 fields of 67^2 x 16 modes
-// 159 us against 40 in LDS, 97^2 x 256 534 against 297, 114^2 x 256 571 against 547.  Only many full planes
-// are faster folded: 129^2 x 128 350 against 329, 129^2 x 256 589 against 654.
+// Whether the unfolded FP64 solve takes less time than the folded FP64 one, whose passes pad a plane's interior
+// n to 2 NH = 128, 256 or 512 and take six launches and more.
+// - Planes in LDS, up to 112 points: always (4 fields of 67^2 x 16 modes 40 us against 159, 97^2 x 256 297
+//   against 534); up to 128, where they fill the padding: up to 128 modes (129^2 x 128 329 against 350,
+//   129^2 x 256 654 against 589).
+// - Passes over the 16s in use, half the padding's products at n^3 = 4 NH^3: up to 9/8 NH always (3 fields of
+//   146^2 x 200 643 us against 1379 folded, one of 140^2 x 8 78 against 88, 3 of 290^2 x 12 313 against 709), up
+//   to 5/4 NH with 64 modes or more (162^2 x 200 836 against 1387; one field of 162^2 x 64 150 against 160, of
+//   162^2 x 16 93 against 91).
+bool unfolded_faster(int n, int nmodes, int NH)
+{
+    if (n <= kPlaneMaxN) return n <= 112 || nmodes <= 128;
+    const int n16 = (n + 15) / 16 * 16;
+    return 8 * n16 <= 9 * NH || (4 * n16 <= 5 * NH && nmodes >= 64);
+}
+
+// Solved without the folded bases.
 bool unfolded_group(const FieldGroup& g, int bidx)
 {
-    return !(L.basis[bidx].NH > 0 && L.fold > bidx) || (plane_supported(g.m, g.m) && (g.n <= 112 || g.nmodes <= 128));
+    const int NH = L.basis[bidx].NH;
+    return !(NH > 0 && L.fold > bidx) || unfolded_faster(g.n, g.nmodes, NH);
 }
 
 int check_group(const FieldGroup& g, int bidx)
@@ -949,6 +963,9 @@ int run_mixed_fold_split(const FieldGroup& g, int bidx, int niter, unsigned long
     return OK;
 }
 
+int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, const char* bounds,
+                 const double* alambda, int m, int nmodes, int ib, double alp, int dir_bmode);
+
 int solve_fields_mixed(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, const char* bounds,
                        const double* alambda, int m, int nmodes, int ib, double alp, int scheme0, int scheme1,
                        int niter, double* stats)
@@ -997,6 +1014,15 @@ int solve_fields_mixed(int nf, const duct_devptr_t* rhs, const duct_devptr_t* so
             return fail(ERR_UNSUPPORTED, "scheme 5 needs a folding basis with ceil((m-2)/2) in (32, 128] "
                         "(m=%d, bound '%c')", m, bidx ? 'n' : 'd');
     }
+    // The unfolded FP64 solve where it is the faster one and no residuals are asked for.  In LDS up to 96 points
+    // (one Dirichlet field of 98^2 x 16 modes 37 us against 44, 3 of 98^2 x 256 208 against 375), and with
+    // Neumann fields, whose low modes take launches of their own, up to 128 (129^2 x 64 'dn' 92 against 189,
+    // 129^2 x 128 'dddn' 329 against 340; Dirichlet fields alone 80 against 59 for one of 129^2 x 64); past the
+    // LDS as for the folded solve (3 fields of 146^2 x 64 239 against 417, one of 162^2 x 64 149 against 152).
+    bool plain = folded && !stats;
+    for (int bidx = 0; bidx < 2; ++bidx)
+        plain = plain && (!gs[bidx].nf || unfolded_faster(gs[bidx].n, nmodes, L.basis[bidx].NH));
+    if (plain && (m - 2 <= 96 || m - 2 > kPlaneMaxN || (gs[1].nf && nmodes <= 128))) return solve_fields(nf, rhs, sol, bounds, alambda, m, nmodes, ib, alp, BND_DIR_ZERO);
     // The folded solve with both groups: the Neumann group on the side stream with its own work
     // arrays, so that its latency-bound kernels (the low modes' FP64 passes, gauge, edges) fill the
     // gaps of the Dirichlet group's (not while launches are timed).

@@ -141,3 +141,41 @@ def test_plane_many_planes_and_folding(dev):
             finally:
                 solver.set_fold(0)
         assert all(np.array_equal(x, y) for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("m,M,bounds", [(67, 3, "d"), (97, 2, "dn"), (98, 3, "ddn"), (130, 4, "dn"), (131, 2, "dn"), (146, 3, "d"),
+                                        (147, 2, "d"), (162, 64, "d")])
+def test_folded_schemes_left_to_unfolded_solves(dev, m, M, bounds):
+    """Where the unfolded FP64 solve is the faster one, the folded solver gives its bits, and so does the refined
+    one (the right-hand sides' Dirichlet walls zeroed alike); with residuals asked for it refines as before."""
+    import torch
+    from duct_amd import solver
+    dev.setup(m)
+    alam = [700.0, 2.0, 1.0][:len(bounds)]
+    f = [field(M, m, 9 * m + k) for k in range(len(bounds))]
+    out = []
+    for kind in ("plain", "fold", "refine", "stats"):
+        rhs = [torch.from_numpy(x).cuda() for x in f]
+        s = [torch.full((M, m, m), float("nan"), dtype=torch.complex128, device="cuda") for _ in f]
+        if kind in ("plain", "fold"):
+            solver.set_fold(0 if kind == "plain" else 2)
+            try:
+                dev.helm3d_batch(rhs, s, bounds, alam, alp=0.9)
+            finally:
+                solver.set_fold(0)
+        else:
+            solver.helm3d_mixed_batch(rhs, s, bounds, alam, alp=0.9, scheme0="fold16q", scheme1="fold16q", niter=1,
+                                      stats=kind == "stats")
+        torch.cuda.synchronize()
+        out.append([x.cpu().numpy() for x in s])
+        after = [r.cpu().numpy() for r in rhs]
+        if kind == "plain":
+            want = after
+        assert all(np.array_equal(a, b) for a, b in zip(after, want))
+    folds = 131 <= m and not (m <= 146 or (m <= 162 and M >= 64))   # m = 147: three modes stay folded
+    for k, x in enumerate(out[0]):
+        assert folds or np.array_equal(out[1][k], x)
+        assert folds or np.array_equal(out[2][k], x)
+        e = [relerr(out[j][k], x) for j in (1, 2, 3)]
+        print("m=%d field %d fold %.2e refine %.2e with stats %.2e" % (m, k, *e), flush=True)
+        assert e[0] <= 1e-11 and e[1] <= 1e-9 and e[2] <= 1e-9
