@@ -98,7 +98,7 @@ struct TempDev {
 struct ShenDev {
     bool ready = false;
     int m = 0;
-    double* frag[4] = {nullptr, nullptr, nullptr, nullptr};   // A_y, A_z, B_y, B_z (m x m padded), k_cline layout
+    double* frag[4] = {nullptr, nullptr, nullptr, nullptr};   // A_y, A_z, B_y, B_z (m x m padded), in fragments (build_frag)
     double* vec = nullptr;                                     // md, mu, sd, lam (n each)
 };
 
@@ -138,7 +138,7 @@ struct Lib {
     size_t tfield_bytes = 0;
     d2v* bscr = nullptr;                  // row sums of the Neumann edge kernels
     size_t bscr_bytes = 0;
-    int dc_m = 0, dc_np = 0;
+    int dc_m = 0;
     int fold = 0;                         // 1: Dirichlet groups use the folded passes, 2: Neumann too
     int fuse_quarters = 1;                // folded passes 2 and 3 on LDS-resident quarters where built
     double* xdft[2] = {nullptr, nullptr}; // advection x-DFTs (inverse, forward), fragment layout
@@ -1504,7 +1504,7 @@ int duct_shutdown_(void)
     free_ptr(L.tfrag[1]);
     for (auto& d : L.dfold) free_ptr(d);
     for (auto& d : L.dfull) free_ptr(d);
-    L.dc_m = L.dc_np = 0;
+    L.dc_m = 0;
     free_ptr(L.rk);
     L.rk_bytes = 0;
     free_temp();
@@ -1689,7 +1689,6 @@ int duct_setup_(const char* bound, const int* m_, const double* P, const double*
             }
         }
         L.dc_m = m;
-        L.dc_np = MP;
     }
     // the interior operator D2B of the solve (pseudomat.f90:110-128, :225-240), column-major
     std::vector<double> op((size_t)n * n, 0.0);
@@ -2269,16 +2268,9 @@ int duct_transyz_dev_(const duct_devptr_t* in, const duct_devptr_t* out, const i
     if ((st = check_common(*m, *nmodes))) return st;
     if (!L.tfrag[0] || L.dc_m != *m)
         return fail(ERR_NOT_SETUP, "no Chebyshev transforms for m=%d (duct_setup_ builds them)", *m);
-    CollocArgs a{};
-    a.g.nf = 1; a.g.nmodes = *nmodes; a.g.m = *m; a.g.n = *m - 2;
-    a.g.in[0] = (const d2v*)*in;
-    a.g.out[0] = (d2v*)*out;
-    a.Dfrag = L.tfrag[*iopt < 0 ? 0 : 1];
-    a.NP = L.dc_np;
-    a.scal = 1.0;
-    a.beta = 0.0;
+    const LineOneArgs a{(const d2v*)*in, (d2v*)*out, L.tfrag[*iopt < 0 ? 0 : 1], 1.0, 0.0, *m, *nmodes, *cdir == 'z'};
     Timed t(PK_DERIV);
-    HIPCHK(launch_colloc(*cdir == 'y' ? CL_DY : CL_DZ, a, L.stream));
+    HIPCHK(launch_line(a, L.stream));
     return OK;
 }
 
@@ -2332,7 +2324,7 @@ int duct_colloc_deriv_dev_(const duct_devptr_t* in, const duct_devptr_t* out, co
     if ((st = check_common(*m, *nmodes))) return st;
     if (!L.dfold[0] || L.dc_m != *m)
         return fail(ERR_NOT_SETUP, "no collocation matrix for m=%d (duct_setup_ builds it)", *m);
-    LineOneArgs a{(const d2v*)*in, (d2v*)*out, L.dfull[*trans ? 2 : 0], *scal, *beta, *m, *nmodes, *cdir == 'z'};
+    const LineOneArgs a{(const d2v*)*in, (d2v*)*out, L.dfull[*trans ? 2 : 0], *scal, *beta, *m, *nmodes, *cdir == 'z'};
     Timed t(PK_DERIV);
     HIPCHK(launch_line(a, L.stream));
     return OK;
@@ -2615,7 +2607,9 @@ int duct_helm3d_temp_dev_(const duct_devptr_t* rhs, const duct_devptr_t* sol, co
     if (!T.ready || T.my != *my || T.mz != *mz)
         return fail(ERR_NOT_SETUP, "duct_setup_temp_ not called for my=%d, mz=%d", *my, *mz);
     const int NP = T.NP, ny = *my - 2, nz = *mz - 2, M = *nmodes;
-    if (plane_supported(*my, *mz)) {
+    // whole solves in LDS, unless the solution lies shifted over the right-hand side (see plane_fields)
+    const uintptr_t fr = *rhs, fs = *sol, fbytes = (uintptr_t)M * *my * *mz * sizeof(d2v);
+    if (plane_supported(*my, *mz) && (fr == fs || fr + fbytes <= fs || fs + fbytes <= fr)) {
         PlaneArgs pa{};
         pa.in[0] = (const d2v*)*rhs;
         pa.out[0] = (d2v*)*sol;
@@ -2707,7 +2701,7 @@ int duct_setup_shen_(const char* bound, const int* m_, const double* Ay, const d
     const int bidx = bound_index(bound[0]);
     if (bidx < 0) return fail(ERR_ARG, "preshen: bound should be d or n, got '%c'", bound[0]);
     const int m = *m_, n = m - 2;
-    if (m < kMinM || m > 16 * 3 * 6) return fail(ERR_UNSUPPORTED, "m=%d outside [%d, 288]", m, kMinM);
+    if (m < kMinM || m > kLineMaxM) return fail(ERR_UNSUPPORTED, "m=%d outside [%d, 288]", m, kMinM);
     int st = ensure_init();
     if (st) return st;
     ShenDev& S = L.shen[bidx];
@@ -2767,16 +2761,9 @@ int duct_helm3d_shen_dev_(const duct_devptr_t* rhs, const duct_devptr_t* sol, co
     if ((st = ensure_buf(L.tfield, L.tfield_bytes, field * sizeof(d2v)))) return st;
     if ((st = ensure_buf(L.sgam, L.sgam_bytes, field * sizeof(double)))) return st;
     auto prod = [&](const d2v* in, d2v* out, int which, bool dirz) -> int {
-        CollocArgs c{};
-        c.g.nf = 1; c.g.nmodes = M; c.g.m = mm; c.g.n = n;
-        c.g.in[0] = in;
-        c.g.out[0] = out;
-        c.Dfrag = S.frag[which];
-        c.NP = (mm + 15) / 16 * 16;
-        c.scal = 1.0;
-        c.beta = 0.0;
+        const LineOneArgs c{in, out, S.frag[which], 1.0, 0.0, mm, M, dirz};
         Timed t(PK_DERIV);
-        HIPCHK(launch_cline(dirz, c, L.stream));
+        HIPCHK(launch_line(c, L.stream));
         return OK;
     };
     d2v* U = (d2v*)*sol;

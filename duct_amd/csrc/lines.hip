@@ -355,8 +355,9 @@ hipError_t launch_lines(const LinesArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
-// ---- one product, unfolded -------------------------------------------------------------------
-// out = coef A u + beta out.  Folding halves the products but rounds each half of the rows at the scale of
+// ---- one product, unfolded: D and D^T, the Chebyshev transforms (transyz), the Shen transforms -------
+// out = coef A u + beta out (derivyz / transyz applied along y or z, chebyshev.f90:1-540, as a dense product with
+// a matrix of the m CGL nodes: pseudomat.f90:90-107, cheb_collocation.F:19-75).  Folding halves the products but rounds each half of the rows at the scale of
 // both: through D and D^T, whose large entries stand at the walls, the gradients of the projection step came
 // out 1.6 times as far off (5.8e-15 against 3.6e-15 at 129^2 x 64), and one product per read is bound by
 // memory or nearly so.  A workgroup owns 16 lines; a wave the row tiles w and w + W, re and im: four

@@ -1,16 +1,11 @@
 // FP64 collocation-operator products on complex(8) fields, v_mfma_f64_16x16x4f64.
 //
 //   k_colloc<CL_RESID>   r = f - (D2B_y u + u D2B_z^T - xlambda u)   interior (n x n)
-//   launch_colloc(CL_DY / CL_DZ): out = beta out + scal (D u | u D^T) on full planes (m x m),
-//                        served by the slab kernel k_cline of deriv.hip
+// (single derivative products on whole planes: k_line of lines.hip)
 //
 // The residual of the mixed solve uses D2B, the interior operator the eigenbasis
 // diagonalises (pseudomat.f90:232-240 Dirichlet, :114-128 Neumann), so r is the
-// residual of exactly the system solvediag solves.  The derivative products
-// apply the collocation derivative matrix DC (pseudomat.f90:90-107, CHQZ
-// (2.4.31), cheb_collocation.F:19-75) or its transpose: d/dy and d/dz of the
-// nodal interpolant, which is what derivyz/transyz compute in coefficient
-// space (chebyshev.f90:1-295, 458-540).
+// residual of exactly the system solvediag solves.
 //
 // Every product accumulates into a register tile whose MFMA row index is z and
 // column index is y, so lanes run along the contiguous y of the field:
@@ -224,8 +219,6 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
 
 hipError_t launch_colloc(int mode, const CollocArgs& a, hipStream_t st)
 {
-    // the single-direction products on whole planes take the slab kernel (deriv.hip)
-    if (mode == CL_DY || mode == CL_DZ) return launch_cline(mode == CL_DZ, a, st);
     const int sz = mode == CL_RESID ? a.g.n : a.g.m;
     const int bpd = (sz + RB - 1) / RB;
     const long nplanes = (long)a.g.nf * a.g.nmodes;
