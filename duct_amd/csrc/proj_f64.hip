@@ -29,13 +29,14 @@
 // (TM*16) x 64 tile in 4*TM v4f64 accumulators.
 //
 // Padding.  Up to seven eighths of the products of a padded plane are with its zeros, and the passes are bound by the
-// FP64 matrix cores (busy 71-81% of the time at 257^2; the rest is stage turnaround that neither wave
-// priorities, a barrier every second stage nor reading a stage's data ahead of its products took away).  From
+// FP64 matrix cores (busy 71-81% of the time at 257^2; the rest is stage turnaround: a wave's burst of products
+// holds the unit that the other wave's stage turn needs.  A barrier every second stage, tiles pipelined over a
+// persistent workgroup and one workgroup of 8 waves did not take it away).  From
 // NP = 256 on (TRIM) a pass therefore computes only the 16s in use: ceil(kn/16) stages, ceil(kn/16) row tiles
 // spread over the waves (TM or TM - 1 each, the larger share rotated over the SIMDs by block), and
 // ceil(cn/16)*16 columns of each plane.  Solves of 4 fields, all of NP -> the 16s in use: 161^2 x 64
-// 1166 -> 420 us, 200^2 x 96 1760 -> 1105, 225^2 x 64 1185 -> 912, 300^2 x 32 4327 -> 1055,
-// 400^2 x 24 3293 -> 1720; full planes the same (257^2 x 256 4.62 ms, 514^2 x 16 2.19).
+// 1166 -> 425 us, 200^2 x 96 1760 -> 1087, 225^2 x 64 1185 -> 912, 300^2 x 32 4327 -> 1055,
+// 400^2 x 24 3293 -> 1720; full planes 4.61 -> 4.55 ms at 257^2 x 256.
 //
 // MFMA lane layout (v_mfma_f64_16x16x4f64, checked by tests/test_gpu_solve.py):
 //   A[i][k] from lane i + 16 k, B[k][j] from lane j + 16 k,
@@ -242,12 +243,22 @@ __global__ __launch_bounds__(256, 2) void k_proj(ProjArgs a)
         if constexpr (TRIM) {
             // a stage count known at run time: two stages per iteration with the fragment buffers swapped (a
             // copy at the loop's end would wait for the loads it rotates in), and the loads of the stage
-            // past the last repeat it (under a branch they would be waited for at once)
+            // past the last repeat it (under a branch they would be waited for at once).  The modes whose stores
+            // into LDS compute (the zeroing of C2P, the divide) take the basis first and run their stage's turn
+            // ahead of the other wave's products: 308 -> 290 and 316 -> 308 us of 512 planes of 257^2; the other
+            // two modes, 281 and 277, gain nothing from either.
             auto stage = [&](int ks, const d2v (&cur)[T][2], d2v (&nxt)[T][2]) {
                 const int kn1 = ks + 1 < NK ? ks + 1 : ks;
-                load_b(kn1);
-                load_a(kn1, nxt);
+                if constexpr (CIN || LDIV) {
+                    load_a(kn1, nxt);
+                    load_b(kn1);
+                    __builtin_amdgcn_s_setprio(0);
+                } else {
+                    load_b(kn1);
+                    load_a(kn1, nxt);
+                }
                 mma(Bs[ks & 1], cur);
+                if constexpr (CIN || LDIV) __builtin_amdgcn_s_setprio(3);
                 store_b((ks & 1) ^ 1, kn1);
                 __syncthreads();
             };
