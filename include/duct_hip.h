@@ -154,7 +154,9 @@ int duct_helm3d_batch_noalloc_dev_(const int *nfields, const duct_devptr_t *rhs,
  * accuracy (scheme0 == scheme1 == 6, niter == 1).  niter in [0, 16].
  * stats (host, may be NULL): (niter+1) x nfields x 2 doubles = max|r| after
  * each step (the last one after the final correction) and max|f|, over the
- * refined modes (schemes 5 and 6: not the FP64-solved low Neumann modes).  */
+ * refined modes (schemes 5 and 6: not the FP64-solved low Neumann modes).
+ * Schemes 5 and 6 without stats are solved in unfolded FP64 at the sizes where
+ * that takes less time (planes far below the folded solve's padded size).    */
 int duct_helm3d_mixed_batch_dev_(const int *nfields, const duct_devptr_t *rhs,
                                  const duct_devptr_t *sol, const char *bounds,
                                  const double *alambda, const int *m, const int *nmodes,
