@@ -2400,9 +2400,10 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     // everything of h but adv and the z derivatives in h; the z launch completes both.
     const double s = -1.0 / (nu * b), gam = gkkc[k], rho = rkkc[k];
     const double sy2 = s * nu * a, sz2 = s * nu * a / (asp * asp);
-    // Where 3 jobs leave CUs idle, adv and h are jobs of their own (h's z job then repeats adv's product),
-    // which shortens the chain of dependent loads and products of a workgroup.
-    // (33^2 x 16 modes: 9.8 + 12.9 against 13.9 + 13.8 us; 97^2 x 40, 728 workgroups: 32.8 + 41.5 against 31.4 + 31.9.)
+    // Small planes take one launch for both directions (k_sums).  Where 3 jobs of larger ones leave CUs idle,
+    // adv and h are jobs of their own (h's z job then repeats adv's product), which shortens the chain of
+    // dependent loads and products of a workgroup.
+    // (At 33^2 x 16 modes 9.8 + 12.9 against 13.9 + 13.8 us, before k_sums took that size; 97^2 x 40, 728 workgroups: 32.8 + 41.5 against 31.4 + 31.9.)
     const bool small = 3L * M * mm < 16 * 256, sums = sums_supported(mm, M);
     if (sums) {
         const double* F1 = L.dfull[0];
