@@ -142,6 +142,8 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
     int q = 0;
     for (int s = 0; s < job.nstage; ++s) {
         const LineStage& st = job.stage[s];
+        // a lone product is scaled after its sum (coef on the matrix rounds every element once more)
+        const bool lone = st.nprod == 1 && (s == 0 || job.stage[s - 1].keep == 0.0);
         for (int pi = 0; pi < st.nprod; ++pi, ++q) {
             const LineProd& p = job.prod[q];
             const bool odd = p.odd != 0;
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
             lds_barrier();                                        // the slab's last readers are done
             store();
             lds_barrier();
-            const double coef = p.coef;
+            const double coef = lone ? 1.0 : p.coef;
             if (odd) {
                 d4v t = ere; ere = ore; ore = t;
                 t = eim; eim = oim; oim = t;
@@ -218,6 +220,13 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
                     ctr[0] += c * S[k];
                     ctr[1] += c * S[2 * SL + k];
                 }
+            }
+            if (lone) {
+                ere *= p.coef;
+                eim *= p.coef;
+                ore *= p.coef;
+                oim *= p.coef;
+                ctr *= p.coef;
             }
         }
 
@@ -564,17 +573,20 @@ __global__ __launch_bounds__(128) void k_sums(SumArgs a)
             }
         }
     };
-    auto mul = [&](auto dir, double coef, const d2v (&u)[2 * KP], const d2v (&f)[KP], d4v& r, d4v& i) {
+    auto mul = [&](auto dir, double coef, const d2v (&u)[2 * KP], const d2v (&f)[KP], d4v& re, d4v& im) {
         constexpr bool Z = decltype(dir)::value;
+        d4v r = {0.0, 0.0, 0.0, 0.0}, i = r;   // (scaled after the sum: coef on f would round every element once more)
 #pragma unroll
         for (int kp = 0; kp < KP; ++kp)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const double d = coef * f[kp][h];
+                const double d = f[kp][h];
                 const d2v x = u[2 * kp + h];
                 r = Z ? mfma(d, x[0], r) : mfma(x[0], d, r);
                 i = Z ? mfma(d, x[1], i) : mfma(x[1], d, i);
             }
+        re += coef * r;
+        im += coef * i;
     };
     auto products = [&](auto dir) {
         constexpr bool Z = decltype(dir)::value;
