@@ -34,8 +34,10 @@ struct LineStage {
     LineTerm term[kLineTerms];
     LineTerm self;
 };
-// A job's stages run in order for each of its lines.  An output may be one of its own stage's terms
-// (read before it is written, at the same point), and no product's source or other job's term.
+// A job's stages run in order for each of its lines; the shares of the centre row (odd m) that a stage passes
+// between the waves are guarded by the barriers of its products, or by one of its own if it has none.  An output
+// may be one of its own stage's terms (read before it is written, at the same point), and no product's source or
+// other job's term.
 struct LineJob {
     LineProd prod[kLineProds];
     LineStage stage[kLineStages];

@@ -233,6 +233,9 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
         // ---- the stage's output: products and terms.  Lane holds rows r (and m-1-r) of 4 lines (y) or
         // 4 rows of one line (z): D[i][j] in lane j + 16 (i % 4), element i / 4.
         if (odd_m) {
+            // the previous stage's shares are read before any wave writes this one's: by the barriers of the
+            // products between, or by one of its own where the stage has no product (the update's U[0] after U[2])
+            if (st.nprod == 0) lds_barrier();
             const d2v c = {ctr[0] + __shfl_xor(ctr[0], 16, 64), ctr[1] + __shfl_xor(ctr[1], 16, 64)};
             const d2v w = {c[0] + __shfl_xor(c[0], 32, 64), c[1] + __shfl_xor(c[1], 32, 64)};
             if (l4 == 0) {
