@@ -530,25 +530,41 @@ bool plane_fields(std::initializer_list<const FieldGroup*> groups)
 
 // Whether the unfolded FP64 solve takes less time than the folded FP64 one, whose passes pad a plane's interior
 // n to 2 NH = 128, 256 or 512 and take six launches and more.
-// - Planes in LDS, up to 112 points: always (4 fields of 67^2 x 16 modes 40 us against 159, 97^2 x 256 297
-//   against 534); up to 128, where they fill the padding: up to 128 modes (129^2 x 128 329 against 350,
-//   129^2 x 256 654 against 589).
-// - Passes over the 16s in use, half the padding's products at n^3 = 4 NH^3: up to 9/8 NH always (3 fields of
-//   146^2 x 200 643 us against 1379 folded, one of 140^2 x 8 78 against 88, 3 of 290^2 x 12 313 against 709), up
-//   to 5/4 NH with 64 modes or more (162^2 x 200 836 against 1387; one field of 162^2 x 64 150 against 160, of
-//   162^2 x 16 93 against 91).
-bool unfolded_faster(int n, int nmodes, int NH)
+// Planes in LDS, `planes` real planes in the launch, `neumann` fields (whose low modes the folded solve gives to
+// launches of their own) among them or not:
+// - up to 112 points always (4 fields of 67^2 x 16 modes 39 us against 159, 97^2 x 256 295 against 557; the
+//   closest is 3 of 113^2 x 64, 123 against 120);
+// - up to 128, where they fill the padding, with Neumann fields up to 1024 planes, four rounds of the 256 CUs
+//   ('dddn' of 130^2 x 128 332 us against 373, 'n' x 512 327 against 421; past it 'dddn' x 192 497 against 490,
+//   x 256 661 against 611);
+// - Dirichlet fields alone from half a round to a whole one ('d' of 130^2 x 64 76 against 76, x 128 82 against
+//   87, 'ddd' x 32 80 against 82; 'd' x 4 74 against 64, and with a second, emptier round 'd' x 192 151 against
+//   121, 'ddd' x 96 220 against 196; with many rounds 'ddd' x 256 455 against 437).
+bool plane_faster(int n, int planes, bool neumann)
 {
-    if (n <= kPlaneMaxN) return n <= 112 || nmodes <= 128;
-    const int n16 = (n + 15) / 16 * 16;
-    return 8 * n16 <= 9 * NH || (4 * n16 <= 5 * NH && nmodes >= 64);
+    if (n <= 112) return true;
+    return neumann ? planes <= 1024 : planes >= 128 && planes <= 256;
 }
 
-// Solved without the folded bases.
-bool unfolded_group(const FieldGroup& g, int bidx)
+// Passes over the 16s in use, half the padding's products at n^3 = 4 NH^3, for a group of `planes` real planes:
+// up to 9/8 NH always (3 fields of 146^2 x 64 modes 238 us against 445 folded, one of 146^2 x 4 76 against 84, 3 of
+// 290^2 x 12 313 against 709), up to 5/4 NH from 128 planes, where the launches are full (162^2 x 200 836
+// against 1387; 3 of 162^2 x 32 154 against 233, one of 162^2 x 64 149 against 160, of 162^2 x 16 92 against 92).
+bool passes_faster(int n, int NH, int planes)
+{
+    const int n16 = (n + 15) / 16 * 16;
+    return 8 * n16 <= 9 * NH || (4 * n16 <= 5 * NH && planes >= 128);
+}
+
+int planes_of(const FieldGroup& g) { return 2 * g.nf * g.nmodes; }
+
+// Solved without the folded bases.  lds: the call's fields may be solved whole in LDS, `planes` and `neumann` of
+// them in one launch (where they may not, a group of up to 128 points takes the folded passes if folding is on).
+bool unfolded_group(const FieldGroup& g, int bidx, bool lds, int planes, bool neumann)
 {
     const int NH = L.basis[bidx].NH;
-    return !(NH > 0 && L.fold > bidx) || unfolded_faster(g.n, g.nmodes, NH);
+    if (!(NH > 0 && L.fold > bidx)) return true;
+    return g.n <= kPlaneMaxN ? lds && plane_faster(g.n, planes, neumann) : passes_faster(g.n, NH, planes_of(g));
 }
 
 int check_group(const FieldGroup& g, int bidx)
@@ -559,13 +575,13 @@ int check_group(const FieldGroup& g, int bidx)
     return OK;
 }
 
-// lds: whole solves in LDS where the group's planes fit (false beside a group whose right-hand sides this
-// one's solutions overlap: they would be written before the other group has read them)
-int run_group(const FieldGroup& g, int bidx, int bmode, bool lds)
+// unfolded: as unfolded_group decided.  lds: whole solves in LDS where the group's planes fit (false beside a group
+// whose right-hand sides this one's solutions overlap: they would be written before the other group has read them)
+int run_group(const FieldGroup& g, int bidx, int bmode, bool unfolded, bool lds)
 {
     int st0 = check_group(g, bidx);
     if (st0) return st0;
-    if (unfolded_group(g, bidx)) return run_group_unfolded(g, bidx, bmode, lds);
+    if (unfolded) return run_group_unfolded(g, bidx, bmode, lds);
     // folded, except the low Poisson modes of a Neumann group (kLowXlam)
     const int klow = bidx == 1 ? low_mode_prefix(g) : 0;
     int st;
@@ -1015,14 +1031,20 @@ int solve_fields_mixed(int nf, const duct_devptr_t* rhs, const duct_devptr_t* so
                         "(m=%d, bound '%c')", m, bidx ? 'n' : 'd');
     }
     // The unfolded FP64 solve where it is the faster one and no residuals are asked for.  In LDS up to 96 points
-    // (one Dirichlet field of 98^2 x 16 modes 37 us against 44, 3 of 98^2 x 256 208 against 375), and with
-    // Neumann fields, whose low modes take launches of their own, up to 128 (129^2 x 64 'dn' 92 against 189,
-    // 129^2 x 128 'dddn' 329 against 340; Dirichlet fields alone 80 against 59 for one of 129^2 x 64); past the
-    // LDS as for the folded solve (3 fields of 146^2 x 64 239 against 417, one of 162^2 x 64 149 against 152).
+    // (one Dirichlet field of 97^2 x 16 modes 37 us against 43, 3 of 97^2 x 256 202 against 370), and with
+    // Neumann fields, whose low modes take launches of their own, as for the folded solve (130^2 x 64 'dn' 94
+    // against 219, 'dddn' of 130^2 x 128 332 against 387; Dirichlet fields alone stay refined: 76 against 58 for
+    // one of 130^2 x 64); past the LDS as for the folded solve (3 fields of 146^2 x 64 238 against 414, one of
+    // 162^2 x 64 149 against 152).
     bool plain = folded && !stats;
-    for (int bidx = 0; bidx < 2; ++bidx)
-        plain = plain && (!gs[bidx].nf || unfolded_faster(gs[bidx].n, nmodes, L.basis[bidx].NH));
-    if (plain && (m - 2 <= 96 || m - 2 > kPlaneMaxN || (gs[1].nf && nmodes <= 128))) return solve_fields(nf, rhs, sol, bounds, alambda, m, nmodes, ib, alp, BND_DIR_ZERO);
+    const int planes = planes_of(gs[0]) + planes_of(gs[1]);
+    if (m - 2 <= kPlaneMaxN) {
+        plain = plain && plane_fields({&gs[0], &gs[1]}) && (m - 2 <= 96 || (gs[1].nf && plane_faster(m - 2, planes, true)));
+    } else {
+        for (int bidx = 0; bidx < 2; ++bidx)
+            plain = plain && (!gs[bidx].nf || passes_faster(m - 2, L.basis[bidx].NH, planes_of(gs[bidx])));
+    }
+    if (plain) return solve_fields(nf, rhs, sol, bounds, alambda, m, nmodes, ib, alp, BND_DIR_ZERO);
     // The folded solve with both groups: the Neumann group on the side stream with its own work
     // arrays, so that its latency-bound kernels (the low modes' FP64 passes, gauge, edges) fill the
     // gaps of the Dirichlet group's (not while launches are timed).
@@ -1155,8 +1177,10 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
         }
     }
     // Planes that fit LDS: every field of both boundary types in one launch.
-    const bool lds = plane_fields({&g[0], &g[1]});
-    if (lds && (!g[0].nf || unfolded_group(g[0], 0)) && (!g[1].nf || unfolded_group(g[1], 1))) {
+    const bool lds = plane_fields({&g[0], &g[1]}), neumann = g[1].nf > 0;
+    const int planes = planes_of(g[0]) + planes_of(g[1]);
+    const bool unfolded[2] = {unfolded_group(g[0], 0, lds, planes, neumann), unfolded_group(g[1], 1, lds, planes, neumann)};
+    if (lds && (!g[0].nf || unfolded[0]) && (!g[1].nf || unfolded[1])) {
         PlaneLaunch p(g[0], dir_bmode);
         for (int bidx = 0; bidx < 2; ++bidx) {
             if (!g[bidx].nf) continue;
@@ -1176,11 +1200,11 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
         }
         HIPCHK(hipEventRecord(L.ev_fork, L.stream));
         HIPCHK(hipStreamWaitEvent(L.side, L.ev_fork, 0));
-        st = run_group(g[0], 0, dir_bmode, lds);
+        st = run_group(g[0], 0, dir_bmode, unfolded[0], lds);
         int st_side;
         {
             SideLane lane;
-            st_side = run_group(g[1], 1, dir_bmode, lds);
+            st_side = run_group(g[1], 1, dir_bmode, unfolded[1], lds);
         }
         HIPCHK(hipEventRecord(L.ev_join, L.side));
         HIPCHK(hipStreamWaitEvent(L.stream, L.ev_join, 0));
@@ -1188,7 +1212,7 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
     }
     for (int bidx = 0; bidx < 2; ++bidx) {
         if (g[bidx].nf == 0) continue;
-        st = run_group(g[bidx], bidx, dir_bmode, lds);
+        st = run_group(g[bidx], bidx, dir_bmode, unfolded[bidx], lds);
         if (st) return st;
     }
     return OK;
@@ -1964,7 +1988,7 @@ static int solve_plane(const char* bound, double xlambda, int imode)
         bc.D2b = B.D2b;
         HIPCHK(launch_bc_correct(bc, L.stream));
     }
-    return run_group(g, bidx, BND_DIR_KEEP, true);
+    return run_group(g, bidx, BND_DIR_KEEP, unfolded_group(g, bidx, true, planes_of(g), bidx == 1), true);
 }
 
 static int plane_buffers(int m)
