@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstring>
 #include <initializer_list>
+#include <map>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -113,6 +114,11 @@ enum ProfKind { PK_C2P = 0, PK_P2P_DIV = 1, PK_GAUGE = 2, PK_P2P = 3, PK_P2C = 4
                 PK_F_P2P_DIV = 17, PK_F_P2P = 18, PK_F_P2C = 19, PK_XPROD = 20, PK_TRIDIAG = 21,
                 PK_F_MID = 22, PK_PLANE = 23 };
 
+struct XdftTables {
+    double* inv = nullptr;   // fragment layout
+    double* fwd = nullptr;
+};
+
 struct Lib {
     bool init = false;
     int device = 0;
@@ -141,11 +147,11 @@ struct Lib {
     int dc_m = 0;
     int fold = 0;                         // 1: Dirichlet groups use the folded passes, 2: Neumann too
     int fuse_quarters = 1;                // folded passes 2 and 3 on LDS-resident quarters where built
-    double* xdft[2] = {nullptr, nullptr}; // advection x-DFTs (inverse, forward), fragment layout
+    // Tables of the x grids, kept per size until duct_shutdown_: a captured graph and a program that alternates
+    // grids go on using theirs.  At most 48 sizes of the dense transforms (10 MB), 120 of k_xprod_fft (2 MB).
+    std::map<std::pair<int, int>, XdftTables> xdft;   // dense x-DFTs by (M, X)
+    std::map<int, d2v*> xtw;              // roots of unity of k_xprod_fft by X (build_xfft_table)
     d2v* xlane = nullptr;                  // twiddles of the 192-point lane FFTs (build_xlane_table)
-    int xdft_M = 0, xdft_X = 0;
-    d2v* xtw = nullptr;                   // roots of unity of k_xprod_fft (build_xfft_table)
-    int xtw_X = 0;
     d2v* prods = nullptr;                 // the six product fields of the advection term
     size_t prods_bytes = 0;
     // x-transforms past the dense kernels' sizes: rocFFT plans (kept per layout), their work
@@ -1218,38 +1224,45 @@ int solve_fields(int nf, const duct_devptr_t* rhs, const duct_devptr_t* sol, con
     return OK;
 }
 
-// The advection x-DFT tables for (M, X), rebuilt when either changes.
-int ensure_xdft(int M, int X)
+// A copy of host data in new device memory
+int upload(double*& dst, const std::vector<double>& src)
 {
-    if (L.xdft_M == M && L.xdft_X == X) return OK;
-    std::vector<double> ei, fw;
-    build_xdft(M, X, ei, fw);
-    HIPCHK(hipStreamSynchronize(L.stream));
-    free_ptr(L.xdft[0]);
-    free_ptr(L.xdft[1]);
-    L.xdft_M = L.xdft_X = 0;
-    HIPCHK(hipMalloc((void**)&L.xdft[0], ei.size() * sizeof(double)));
-    HIPCHK(hipMemcpy(L.xdft[0], ei.data(), ei.size() * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMalloc((void**)&L.xdft[1], fw.size() * sizeof(double)));
-    HIPCHK(hipMemcpy(L.xdft[1], fw.data(), fw.size() * sizeof(double), hipMemcpyHostToDevice));
-    L.xdft_M = M;
-    L.xdft_X = X;
+    HIPCHK(hipMalloc((void**)&dst, src.size() * sizeof(double)));
+    const hipError_t e = hipMemcpy(dst, src.data(), src.size() * sizeof(double), hipMemcpyHostToDevice);
+    if (e != hipSuccess) free_ptr(dst);
+    HIPCHK(e);
     return OK;
 }
 
-// The roots of unity of the X-point transforms of k_xprod_fft, rebuilt when X changes.
-int ensure_xtw(int X)
+// The x-DFT tables of the dense transforms for (M, X), built at the first call with these sizes.
+int ensure_xdft(int M, int X, XdftTables& t)
 {
-    if (L.xtw_X == X) return OK;
-    std::vector<double> tab;
-    build_xfft_table(X, tab);
-    HIPCHK(hipStreamSynchronize(L.stream));
-    free_ptr(L.xtw);
-    L.xtw_X = 0;
-    HIPCHK(hipMalloc((void**)&L.xtw, tab.size() * sizeof(double)));
-    HIPCHK(hipMemcpy(L.xtw, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
-    L.xtw_X = X;
-    return OK;
+    XdftTables& kept = L.xdft[{M, X}];
+    int st = OK;
+    if (!kept.inv || !kept.fwd) {
+        std::vector<double> ei, fw;
+        build_xdft(M, X, ei, fw);
+        if (!kept.inv) st = upload(kept.inv, ei);
+        if (!st) st = upload(kept.fwd, fw);
+    }
+    t = kept;
+    return st;
+}
+
+// The roots of unity of the X-point transforms of k_xprod_fft, built at the first call with this X.
+int ensure_xtw(int X, const d2v*& t)
+{
+    d2v*& kept = L.xtw[X];
+    int st = OK;
+    if (!kept) {
+        std::vector<double> tab;
+        build_xfft_table(X, tab);
+        double* p = nullptr;
+        st = upload(p, tab);
+        kept = (d2v*)p;
+    }
+    t = kept;
+    return st;
 }
 
 // One launch of derivative sums (lines.hip) on the library's stream.
@@ -1432,22 +1445,24 @@ int xprods_run(const d2v* const in[3], int mm, int M, int X)
         Timed t(PK_XPROD);
         HIPCHK(launch_xprod_lane(xa, L.xlane, L.stream));
     } else if (xprod_fft_supported(M, X) && !(dense_x(M, X) && M * X <= 1024)) {
-        if ((st = ensure_xtw(X))) return st;
+        const d2v* tw = nullptr;
+        if ((st = ensure_xtw(X, tw))) return st;
         XprodArgs xa{};
         for (int i = 0; i < 3; ++i) xa.in[i] = in[i];
         for (int p = 0; p < 6; ++p) xa.out[p] = L.prods + p * field;
         xa.m = mm; xa.M = M; xa.X = X;
         Timed t(PK_XPROD);
-        HIPCHK(launch_xprod_fft(xa, L.xtw, L.stream));
+        HIPCHK(launch_xprod_fft(xa, tw, L.stream));
     } else if (!dense_x(M, X)) {
         if ((st = xprod_fft(in, L.prods, mm, M, X))) return st;
     } else {
-        if ((st = ensure_xdft(M, X))) return st;
+        XdftTables dft;
+        if ((st = ensure_xdft(M, X, dft))) return st;
         XprodArgs xa{};
         for (int i = 0; i < 3; ++i) xa.in[i] = in[i];
         for (int p = 0; p < 6; ++p) xa.out[p] = L.prods + p * field;
-        xa.Einv = L.xdft[0];
-        xa.Fwd = L.xdft[1];
+        xa.Einv = dft.inv;
+        xa.Fwd = dft.fwd;
         xa.m = mm; xa.M = M; xa.X = X;
         Timed t(PK_XPROD);
         HIPCHK(launch_xprod(xa, L.stream));
@@ -1540,11 +1555,13 @@ int duct_shutdown_(void)
     free_ptr(L.bscr);
     L.bscr_bytes = 0;
     free_ptr(L.xlane);
-    free_ptr(L.xtw);
-    L.xtw_X = 0;
-    free_ptr(L.xdft[0]);
-    free_ptr(L.xdft[1]);
-    L.xdft_M = L.xdft_X = 0;
+    for (auto& t : L.xtw) free_ptr(t.second);
+    L.xtw.clear();
+    for (auto& t : L.xdft) {
+        free_ptr(t.second.inv);
+        free_ptr(t.second.fwd);
+    }
+    L.xdft.clear();
     free_ptr(L.prods);
     L.prods_bytes = 0;
     for (auto& xp : L.xplans) (void)rocfft_plan_destroy(xp.plan);
@@ -2240,12 +2257,13 @@ int duct_fourx_dev_(const duct_devptr_t* fou, const duct_devptr_t* phys, const i
         }
         return OK;
     }
-    if ((st = ensure_xdft(M, X))) return st;
+    XdftTables tab;
+    if ((st = ensure_xdft(M, X, tab))) return st;
     FourxArgs a{};
     a.fou = (d2v*)*fou;
     a.phys = (double*)*phys;
-    a.Einv = L.xdft[0];
-    a.Fwd = L.xdft[1];
+    a.Einv = tab.inv;
+    a.Fwd = tab.fwd;
     a.lines = lines;
     a.M = M; a.X = X; a.inverse = *iopt >= 0;
     Timed t(PK_XPROD);
