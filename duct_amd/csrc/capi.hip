@@ -1428,9 +1428,10 @@ int xprods_run(const d2v* const in[3], int mm, int M, int X)
     const size_t field = (size_t)M * mm * mm;
     if ((st = ensure_buf(L.prods, L.prods_bytes, 6 * field * sizeof(d2v)))) return st;
     // X = 192 and M <= 64: 64-point FFTs across DPP rows (62 us at 129^2 x 64 modes against 83 of
-    // k_xprod_fft); other even X of factors 2, 3 and 5: FFTs through LDS; the remaining sizes (X with
-    // another factor) and the smallest grids (M X <= 1024: 13.5 us at 33^2 x 16 modes, mgalx 48, against
-    // 14.0; at 32 x 96 it is 38 against 26) as dense transforms where those are built, else rocFFT.
+    // k_xprod_fft); other even X of factors 2, 3 and 5: FFTs through LDS; X with another factor as dense
+    // transforms where those are built, else rocFFT.  (Dense against FFT, a whole advection call: 16 modes and
+    // X = 48 16.4 us against 17.4 at 33^2, 49 against 47 at 97^2, 222 against 171 at 257^2; X = 64 17.9 against
+    // 17.6 at 33^2, 53 against 48 at 97^2; 32 modes and X = 96 25.6 against 21.4 at 33^2, 87 against 59 at 97^2.)
     if (X == 192 && M <= 64) {
         if (!L.xlane) {
             std::vector<double> tab;
@@ -1444,7 +1445,7 @@ int xprods_run(const d2v* const in[3], int mm, int M, int X)
         xa.m = mm; xa.M = M; xa.X = X;
         Timed t(PK_XPROD);
         HIPCHK(launch_xprod_lane(xa, L.xlane, L.stream));
-    } else if (xprod_fft_supported(M, X) && !(dense_x(M, X) && M * X <= 1024)) {
+    } else if (xprod_fft_supported(M, X)) {
         const d2v* tw = nullptr;
         if ((st = ensure_xtw(X, tw))) return st;
         XprodArgs xa{};
