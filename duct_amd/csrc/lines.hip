@@ -140,10 +140,24 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
     d4v ere = {0.0, 0.0, 0.0, 0.0}, eim = ere, ore = ere, oim = ere;   // E and O of the wave's row tile
     d2v ctr = {0.0, 0.0};                                              // this thread's share of the centre row
     int q = 0;
+    // The accumulators hold the sums over `unit`, the last product's coef: coef on the matrix rounds every element
+    // once more (p's median error over 24 steps of 97^2 x 40 modes 2.64e-13 with it, 2.54e-13 without; 129^2 x 64
+    // 4.07e-13 and 4.00e-13; the time is the same to 0.7%).
+    auto rescale = [&](double f) {
+        ere *= f;
+        eim *= f;
+        ore *= f;
+        oim *= f;
+        ctr *= f;
+    };
     for (int s = 0; s < job.nstage; ++s) {
         const LineStage& st = job.stage[s];
-        // a lone product is scaled after its sum (coef on the matrix rounds every element once more)
-        const bool lone = st.nprod == 1 && (s == 0 || job.stage[s - 1].keep == 0.0);
+        double unit = 1.0;
+        bool empty = s == 0 || job.stage[s - 1].keep == 0.0;
+        if (empty) {   // (0 times the previous output is not zero where that is infinite)
+            ere = eim = ore = oim = d4v{0.0, 0.0, 0.0, 0.0};
+            ctr = d2v{0.0, 0.0};
+        }
         for (int pi = 0; pi < st.nprod; ++pi, ++q) {
             const LineProd& p = job.prod[q];
             const bool odd = p.odd != 0;
@@ -154,7 +168,10 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
             lds_barrier();                                        // the slab's last readers are done
             store();
             lds_barrier();
-            const double coef = lone ? 1.0 : p.coef;
+            if (p.coef == 0.0) continue;                          // (1 / aspect at its limit) nothing to add
+            if (!empty) rescale(unit / p.coef);
+            unit = p.coef;
+            empty = false;
             if (odd) {
                 d4v t = ere; ere = ore; ore = t;
                 t = eim; eim = oim; oim = t;
@@ -169,7 +186,7 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
                 for (int h = 0; h < 2; ++h) {
                     const double* S = S0 + (2 * kp + h) * 4;
                     const double er = S[0], orr = S[SL], ei = S[2 * SL], oi = S[3 * SL];
-                    const double dp = coef * cp[h], dm = coef * cm[h];
+                    const double dp = cp[h], dm = cm[h];
                     if constexpr (!DIRZ) {
                         ere = mfma(er, dp, ere);
                         eim = mfma(ei, dp, eim);
@@ -198,7 +215,7 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
                 for (int h = 0; h < 2; ++h) {
                     const double* S = S0 + (2 * KPO + h) * 4;
                     const double er = S[0], ei = S[2 * SL];
-                    const double dp = coef * fp[h];
+                    const double dp = fp[h];
                     if constexpr (!DIRZ) {
                         ere = mfma(er, dp, ere);
                         eim = mfma(ei, dp, eim);
@@ -216,19 +233,13 @@ __global__ __launch_bounds__(576, 4) void k_lines(LinesArgs a, int nslab)
                 const double* C = p.mat + (size_t)2 * KH * KH;
                 const double* S = slab + (odd ? SL : 0) + l16 * LDK;
                 for (int k = tid >> 4; k < he; k += nth >> 4) {
-                    const double c = coef * C[k];
+                    const double c = C[k];
                     ctr[0] += c * S[k];
                     ctr[1] += c * S[2 * SL + k];
                 }
             }
-            if (lone) {
-                ere *= p.coef;
-                eim *= p.coef;
-                ore *= p.coef;
-                oim *= p.coef;
-                ctr *= p.coef;
-            }
         }
+        if (st.nprod > 0) rescale(unit);
 
         // ---- the stage's output: products and terms.  Lane holds rows r (and m-1-r) of 4 lines (y) or
         // 4 rows of one line (z): D[i][j] in lane j + 16 (i % 4), element i / 4.

@@ -54,3 +54,22 @@ def test_substeps_on_odd_grids(dev, oracle_mod, m, M, aspect):
                 assert max(e) <= (1e-10 * max(1.0, (m / 129.0) ** 4) if name == "p" else 1e-10)
     finally:
         oracle_mod.use_blas(False)
+
+
+@pytest.mark.parametrize("m,M", [(65, 4), (65, 24)])
+def test_substep_without_z_derivatives(dev, oracle_mod, m, M):
+    """aspect = inf: 1 / aspect is zero, and so are the coefficients of the z products, some of which join sums that
+    others have begun."""
+    import torch
+    from duct_amd import step
+    from oracle import rk3 as R
+    fnu, dt, alp, dpdx, X = 0.01, 0.02, 0.9, 0.3, 3 * M
+    dev.setup(m)
+    fields, adv = initial_state(m, M, m)
+    F, A = ([torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in g] for g in (fields, adv))
+    step.rk3_substep(*F, A, 2, fnu, dt, X, alp=alp, aspect=float("inf"), dpdx=dpdx)
+    torch.cuda.synchronize()
+    ref = R.rk3_substep(*fields, tuple(adv), 2, fnu, dt, X, oracle_helm(oracle_mod, m, alp), alp, aspect=float("inf"), dpdx=dpdx)
+    errs = [relerr(g.cpu().numpy(), r) for g, r in zip(F + A, list(ref[:4]) + list(ref[4]))]
+    print("m=%d M=%d aspect=inf rel.err %s" % (m, M, " ".join("%.1e" % e for e in errs)), flush=True)
+    assert max(errs) <= 1e-10
