@@ -2446,7 +2446,9 @@ int duct_rk3_substep_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const 
     // Small planes take one launch for both directions (k_sums).  Where 3 jobs of larger ones leave CUs idle,
     // adv and h are jobs of their own (h's z job then repeats adv's product), which shortens the chain of
     // dependent loads and products of a workgroup.
-    // (At 33^2 x 16 modes 9.8 + 12.9 against 13.9 + 13.8 us, before k_sums took that size; 97^2 x 40, 728 workgroups: 32.8 + 41.5 against 31.4 + 31.9.)
+    // (A step with jobs of their own against without: 65^2 x 4 modes 322 us against 367, 65^2 x 20 392 against 417,
+    // 97^2 x 8 551 against 586, 129^2 x 8 805 against 847, 257^2 x 5 1723 against 1781; past the line, 97^2 x 40, the
+    // two launches of the right-hand sides 32.8 + 41.5 us against 31.4 + 31.9.)
     const bool small = 3L * M * mm < 16 * 256, sums = sums_supported(mm, M);
     if (sums) {
         const double* F1 = L.dfull[0];
