@@ -2655,7 +2655,7 @@ int duct_helm3d_temp_dev_(const duct_devptr_t* rhs, const duct_devptr_t* sol, co
     const int NP = T.NP, ny = *my - 2, nz = *mz - 2, M = *nmodes;
     // whole solves in LDS, unless the solution lies shifted over the right-hand side (see plane_fields)
     const uintptr_t fr = *rhs, fs = *sol, fbytes = (uintptr_t)M * *my * *mz * sizeof(d2v);
-    if (plane_supported(*my, *mz) && (fr == fs || fr + fbytes <= fs || fs + fbytes <= fr)) {
+    if (plane_supported(*my, *mz) && (fr + fbytes <= fs || fs + fbytes <= fr)) {
         PlaneArgs pa{};
         pa.in[0] = (const d2v*)*rhs;
         pa.out[0] = (d2v*)*sol;

@@ -1,6 +1,6 @@
 // FP64 collocation-operator products on complex(8) fields, v_mfma_f64_16x16x4f64.
 //
-//   k_colloc<CL_RESID>   r = f - (D2B_y u + u D2B_z^T - xlambda u)   interior (n x n)
+//   k_colloc   r = f - (D2B_y u + u D2B_z^T - xlambda u)   interior (n x n)
 // (single derivative products on whole planes: k_line of lines.hip)
 //
 // The residual of the mixed solve uses D2B, the interior operator the eigenbasis
@@ -35,16 +35,10 @@ __device__ __forceinline__ void atomic_max_pos(unsigned long long* p, double v)
 }
 }  // namespace
 
-template <int MODE>
-__global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long nplanes)
+__global__ __launch_bounds__(256, 2) void k_colloc(ResidArgs a, int bpd, long nplanes)
 {
-    constexpr bool RESID = MODE == CL_RESID;
-    constexpr bool YT = MODE != CL_DZ;   // y term present
-    constexpr bool ZT = MODE != CL_DY;   // z term present
     const FieldGroup& g = a.g;
-    const int NP = a.NP, m = g.m;
-    const int off = RESID ? 1 : 0;            // interior or full plane
-    const int sz = RESID ? g.n : m;
+    const int NP = a.NP, m = g.m, sz = g.n;
     // XCD-aware numbering: 8 consecutive planes share a group of 8*bpd^2 ids,
     // plane = group*8 + id%8, block = (id/8) % bpd^2.
     const long bid = blockIdx.x;
@@ -55,12 +49,10 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
     if (plane >= nplanes) return;
     const int f = (int)(plane / g.nmodes), mode = (int)(plane % g.nmodes);
     const int z0 = (blk / bpd) * RB, y0 = (blk % bpd) * RB;
-    // RESID: g.out = current solution u, g.in = right-hand side f.
-    // DY/DZ: g.in = operand, g.out = result.
-    const d2v* U = (RESID ? (const d2v*)g.out[f] : g.in[f]) + (size_t)mode * m * m;
+    const d2v* U = (const d2v*)g.out[f] + (size_t)mode * m * m;
 
-    __shared__ double Uz[ZT ? 2 : 1][2][ZT ? RB * RLD : 1];   // [buf][re/im][y][k]: u(y0+y, k0+k)
-    __shared__ double Uy[YT ? 2 : 1][2][YT ? RB * RLD : 1];   // [buf][re/im][z][k]: u(k0+k, z0+z)
+    __shared__ double Uz[2][2][RB * RLD];   // [buf][re/im][y][k]: u(y0+y, k0+k)
+    __shared__ double Uy[2][2][RB * RLD];   // [buf][re/im][z][k]: u(k0+k, z0+z)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, l4 = lane >> 4;
@@ -76,27 +68,19 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
         const int k0 = ks * RKT;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if constexpr (ZT) {
-                const int y = y0 + uz_y + e, kz = k0 + uz_k;
-                rz[e] = (y < sz && kz < sz) ? U[(size_t)(y + off) + (size_t)(kz + off) * m] : d2v{0.0, 0.0};
-            }
-            if constexpr (YT) {
-                const int z = z0 + uy_z, ky = k0 + uy_k + e;
-                ry[e] = (z < sz && ky < sz) ? U[(size_t)(ky + off) + (size_t)(z + off) * m] : d2v{0.0, 0.0};
-            }
+            const int y = y0 + uz_y + e, kz = k0 + uz_k;
+            rz[e] = (y < sz && kz < sz) ? U[(size_t)(y + 1) + (size_t)(kz + 1) * m] : d2v{0.0, 0.0};
+            const int z = z0 + uy_z, ky = k0 + uy_k + e;
+            ry[e] = (z < sz && ky < sz) ? U[(size_t)(ky + 1) + (size_t)(z + 1) * m] : d2v{0.0, 0.0};
         }
     };
     auto store = [&](int buf) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if constexpr (ZT) {
-                Uz[buf][0][(uz_y + e) * RLD + uz_k] = rz[e][0];
-                Uz[buf][1][(uz_y + e) * RLD + uz_k] = rz[e][1];
-            }
-            if constexpr (YT) {
-                Uy[buf][0][uy_z * RLD + uy_k + e] = ry[e][0];
-                Uy[buf][1][uy_z * RLD + uy_k + e] = ry[e][1];
-            }
+            Uz[buf][0][(uz_y + e) * RLD + uz_k] = rz[e][0];
+            Uz[buf][1][(uz_y + e) * RLD + uz_k] = rz[e][1];
+            Uy[buf][0][uy_z * RLD + uy_k + e] = ry[e][0];
+            Uy[buf][1][uy_z * RLD + uy_k + e] = ry[e][1];
         }
     };
 
@@ -128,8 +112,8 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                if constexpr (ZT) az[t][h] = dfrag(zt0 + t, ks * 2 + h);
-                if constexpr (YT) by[t][h] = dfrag(yt0 + t, ks * 2 + h);
+                az[t][h] = dfrag(zt0 + t, ks * 2 + h);
+                by[t][h] = dfrag(yt0 + t, ks * 2 + h);
             }
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
@@ -139,19 +123,17 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
                 double bu[2], au[2];
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    if constexpr (ZT) bu[t] = Uz[buf][p][(wy * 32 + t * 16 + l16) * RLD + kl];   // B[k][y] = u(y,k)
-                    if constexpr (YT) au[t] = Uy[buf][p][(wz * 32 + t * 16 + l16) * RLD + kl];   // A[z][k] = u(k,z)
+                    bu[t] = Uz[buf][p][(wy * 32 + t * 16 + l16) * RLD + kl];   // B[k][y] = u(y,k)
+                    au[t] = Uy[buf][p][(wz * 32 + t * 16 + l16) * RLD + kl];   // A[z][k] = u(k,z)
                 }
 #pragma unroll
                 for (int zt = 0; zt < 2; ++zt)
 #pragma unroll
                     for (int yt = 0; yt < 2; ++yt) {
-                        if constexpr (ZT)
-                            acc[zt][yt][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                az[zt][kk >> 1][kk & 1], bu[yt], acc[zt][yt][p], 0, 0, 0);
-                        if constexpr (YT)
-                            acc[zt][yt][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                                au[zt], by[yt][kk >> 1][kk & 1], acc[zt][yt][p], 0, 0, 0);
+                        acc[zt][yt][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            az[zt][kk >> 1][kk & 1], bu[yt], acc[zt][yt][p], 0, 0, 0);
+                        acc[zt][yt][p] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            au[zt], by[yt][kk >> 1][kk & 1], acc[zt][yt][p], 0, 0, 0);
                     }
             }
         }
@@ -160,79 +142,54 @@ __global__ __launch_bounds__(256, 2) void k_colloc(CollocArgs a, int bpd, long n
     }
 
     // epilogue: D[i=z][j=y] in lane j + 16 (i%4), element i/4
-    if constexpr (RESID) {
-        const d2v* F = g.in[f] + (size_t)mode * m * m;
-        const double xlam = xlambda_of(g.alambda[f], g.alp, g.mode0 + mode);
-        const bool zim = (g.mode0 + mode) == 0;
-        const bool singular = a.neumann && fabs(xlam) <= 1.0e-10;
-        d2v* R = a.r[f] + (size_t)mode * m * m;
-        double rmx = 0.0, fmx = 0.0;
+    const d2v* F = g.in[f] + (size_t)mode * m * m;
+    const double xlam = xlambda_of(g.alambda[f], g.alp, g.mode0 + mode);
+    const bool zim = (g.mode0 + mode) == 0;
+    const bool singular = a.neumann && fabs(xlam) <= 1.0e-10;
+    d2v* R = a.r[f] + (size_t)mode * m * m;
+    double rmx = 0.0, fmx = 0.0;
 #pragma unroll
-        for (int zt = 0; zt < 2; ++zt)
+    for (int zt = 0; zt < 2; ++zt)
 #pragma unroll
-            for (int yt = 0; yt < 2; ++yt)
+        for (int yt = 0; yt < 2; ++yt)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int z = z0 + wz * 32 + zt * 16 + 4 * e + l4;
-                    const int y = y0 + wy * 32 + yt * 16 + l16;
-                    if (z < sz && y < sz) {
-                        const size_t idx = (size_t)(y + 1) + (size_t)(z + 1) * m;
-                        const d2v u = U[idx], fv = F[idx];
-                        d2v lu = {acc[zt][yt][0][e], acc[zt][yt][1][e]};
-                        d2v rv = fv - (lu - xlam * u);
-                        if (zim) rv[1] = 0.0;
-                        R[idx] = rv;
-                        if (!singular) rmx = fmax(rmx, fmax(fabs(rv[0]), fabs(rv[1])));
-                        fmx = fmax(fmx, fmax(fabs(fv[0]), zim ? 0.0 : fabs(fv[1])));
-                    }
+            for (int e = 0; e < 4; ++e) {
+                const int z = z0 + wz * 32 + zt * 16 + 4 * e + l4;
+                const int y = y0 + wy * 32 + yt * 16 + l16;
+                if (z < sz && y < sz) {
+                    const size_t idx = (size_t)(y + 1) + (size_t)(z + 1) * m;
+                    const d2v u = U[idx], fv = F[idx];
+                    d2v lu = {acc[zt][yt][0][e], acc[zt][yt][1][e]};
+                    d2v rv = fv - (lu - xlam * u);
+                    if (zim) rv[1] = 0.0;
+                    R[idx] = rv;
+                    if (!singular) rmx = fmax(rmx, fmax(fabs(rv[0]), fabs(rv[1])));
+                    fmx = fmax(fmx, fmax(fabs(fv[0]), zim ? 0.0 : fabs(fv[1])));
                 }
-        if (a.stats) {
+            }
+    if (a.stats) {
 #pragma unroll
-            for (int sh = 32; sh > 0; sh >>= 1) {
-                rmx = fmax(rmx, __shfl_xor(rmx, sh, 64));
-                fmx = fmax(fmx, __shfl_xor(fmx, sh, 64));
-            }
-            if (lane == 0) {
-                atomic_max_pos(a.stats + 2 * a.slot[f], rmx);
-                atomic_max_pos(a.stats + 2 * a.slot[f] + 1, fmx);
-            }
+        for (int sh = 32; sh > 0; sh >>= 1) {
+            rmx = fmax(rmx, __shfl_xor(rmx, sh, 64));
+            fmx = fmax(fmx, __shfl_xor(fmx, sh, 64));
         }
-    } else {
-        d2v* O = g.out[f] + (size_t)mode * m * m;
-#pragma unroll
-        for (int zt = 0; zt < 2; ++zt)
-#pragma unroll
-            for (int yt = 0; yt < 2; ++yt)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int z = z0 + wz * 32 + zt * 16 + 4 * e + l4;
-                    const int y = y0 + wy * 32 + yt * 16 + l16;
-                    if (z < sz && y < sz) {
-                        const size_t idx = (size_t)y + (size_t)z * m;
-                        d2v v = {a.scal * acc[zt][yt][0][e], a.scal * acc[zt][yt][1][e]};
-                        if (a.beta != 0.0) v += a.beta * O[idx];
-                        O[idx] = v;
-                    }
-                }
+        if (lane == 0) {
+            atomic_max_pos(a.stats + 2 * a.slot[f], rmx);
+            atomic_max_pos(a.stats + 2 * a.slot[f] + 1, fmx);
+        }
     }
 }
 
-hipError_t launch_colloc(int mode, const CollocArgs& a, hipStream_t st)
+hipError_t launch_resid(const ResidArgs& a, hipStream_t st)
 {
-    const int sz = mode == CL_RESID ? a.g.n : a.g.m;
-    const int bpd = (sz + RB - 1) / RB;
+    const int bpd = (a.g.n + RB - 1) / RB;
     const long nplanes = (long)a.g.nf * a.g.nmodes;
     const long groups = (nplanes + kXcd - 1) / kXcd;
     const long blocks = groups * kXcd * bpd * bpd;
     if (blocks <= 0) return hipSuccess;
-    switch (mode) {
-        case CL_RESID: hipLaunchKernelGGL(k_colloc<CL_RESID>, dim3((unsigned)blocks), dim3(256), 0, st, a, bpd, nplanes); break;
-        default: return hipErrorInvalidValue;
-    }
+    hipLaunchKernelGGL(k_colloc, dim3((unsigned)blocks), dim3(256), 0, st, a, bpd, nplanes);
     return hipGetLastError();
 }
-
-hipError_t launch_resid(const ResidArgs& a, hipStream_t st) { return launch_colloc(CL_RESID, a, st); }
 
 // out = beta out + scal * (i alp k) in, k = mode0 + mode  (derivx, fourier.F:117-188, ider=1)
 __global__ __launch_bounds__(256) void k_derivx(const d2v* __restrict__ in, d2v* out, long mm, int nmodes, int mode0,
