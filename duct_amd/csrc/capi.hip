@@ -511,15 +511,18 @@ struct PlaneLaunch {
     }
 };
 
-// A launch of whole solves reads a plane and writes its solution while others are still to be read: a
-// solution may be its own right-hand side but overlap no other field (the projection passes read every
-// right-hand side before they write a solution, so those fields keep them).
+// A launch of whole solves reads a plane, writes its solution and may zero its right-hand side's walls while others
+// are still to be read: a solution may be its own right-hand side but overlap no other field, and right-hand sides
+// may share whole planes only, whose walls are walls to both (the projection passes read every right-hand side
+// before they write, so those fields keep them).
 bool plane_fields(std::initializer_list<const FieldGroup*> groups)
 {
     std::vector<std::pair<uintptr_t, uintptr_t>> in, out;
+    uintptr_t plane = 1;   // bytes of a complex plane, the same for all groups
     for (const FieldGroup* g : groups) {
         if (!plane_supported(g->m, g->m)) return false;
-        const uintptr_t bytes = (uintptr_t)g->nmodes * g->m * g->m * sizeof(d2v);
+        plane = (uintptr_t)g->m * g->m * sizeof(d2v);
+        const uintptr_t bytes = g->nmodes * plane;
         for (int f = 0; f < g->nf; ++f) {
             in.emplace_back((uintptr_t)g->in[f], (uintptr_t)g->in[f] + bytes);
             out.emplace_back((uintptr_t)g->out[f], (uintptr_t)g->out[f] + bytes);
@@ -530,6 +533,7 @@ bool plane_fields(std::initializer_list<const FieldGroup*> groups)
         for (size_t j = 0; j < in.size(); ++j) {
             if (meet(out[i], in[j]) && !(i == j && out[i].first == in[j].first)) return false;
             if (i != j && meet(out[i], out[j])) return false;
+            if (in[i].first < in[j].first && meet(in[i], in[j]) && (in[j].first - in[i].first) % plane) return false;
         }
     return true;
 }
