@@ -79,9 +79,11 @@ def _check_field(t, m: int):
 
 def _use_current_stream():
     # the handle of torch.cuda.current_stream() without its Stream object: 0.9 us instead of 3.4, which a call of
-    # helm3d_batch on a small grid waits for (12.9 us, now 9.0; its kernel takes 7)
+    # helm3d_batch on a small grid waits for (12.9 us, now 9.0; its kernel takes 7).  A private name of torch: where
+    # a release has it not, the public way.
     import torch
-    set_stream(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    set_stream(raw(torch.cuda.current_device()) if raw else torch.cuda.current_stream().cuda_stream)
 
 
 def helm3d(rhs, sol, bound: str, alambda: float, alp: float = 1.0, ib: int = 0) -> None:
