@@ -24,8 +24,7 @@
 // of 17 MB each (the y launch's sums go through memory to the z launch) in 87 and 95 us, 3.6-3.8
 // TB/s where a copy reaches 4.4-5.1; at 257^2 x 128 modes 816 and 878 us, 3.2 TB/s with the MFMAs
 // busy half the time.  All derivative and elementwise work of an RK3 step took 1537 us at 129^2 x 64
-// as nine launches per substep and takes 870 us as six; at 257^2 x 128, 12800 and 7500 us.
-//
+// as nine launches per substep and takes 888 us as six; at 257^2 x 128, 12800 and 7800 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -541,7 +540,7 @@ hipError_t launch_line(const LineOneArgs& a, hipStream_t st)
 // issued before the first product; the planes are a few KB and come from the caches), no staging and one
 // barrier, where the second wave's sums join the first's.  Nothing is folded: at these sizes the products are
 // a third of a workgroup's time.  A 33^2 x 16 step of 27 launches took 251 us, of these 18 y and z launches;
-// with 9 of k_sums it takes 141 us.
+// with 9 of k_sums it takes 139 us.
 template <int KP, int NPR>
 __global__ __launch_bounds__(128) void k_sums(SumArgs a)
 {

@@ -20,9 +20,9 @@
 //
 // What bounds it: the FP64 matrix cores.  At RT = 8 a plane takes ~155e3 cycles of which its MFMAs are
 // 131e3; the rest is what one workgroup per CU cannot overlap: the writes between the passes (~4e3
-// each), the divide (~9e3), the stores and walls.  u, v, w and p at 129^2 x 64 modes take 170 us
+// each), the divide (~9e3), the stores and walls.  u, v, w and p at 129^2 x 64 modes take 173 us
 // (8 launches and 216 us as passes over planar intermediates), at 129^2 x 256 652 us (736), one field of
-// 33^2 x 16 11 us (31), 97^2 x 40 51 us for the Neumann field, the mixed walls at 97 x 129 x 64 81 us (140)
+// 33^2 x 16 9 us (31), 97^2 x 40 51 us for the Neumann field, the mixed walls at 97 x 129 x 64 81 us (140)
 // and at 129 x 129 x 400 362 us (483).
 #include <algorithm>
 

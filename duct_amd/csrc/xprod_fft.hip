@@ -6,16 +6,16 @@
 // What bounds it: the nine fields of M modes per line cross HBM once, 9 x 16 B x M per line, and
 // everything else happens in registers and LDS.
 //
-// Two neighbouring lines share a complex transform, for each of u, v, w and each product, so a line
-// costs 1.5 inverse and 3 forward complex transforms of X points.  (Sharing it between u and v of a line,
-// and between uu and vv, leaves the rounding of the larger in the smaller: at 384 x 128 x 257^2 the v and w
-// components of a duct flow's advection were 7.9e-15 and 6.4e-15 off, now 5.3e-15 and 5.4e-15; with rocFFT's
-// transforms of one real line each 5.6e-15 and 5.5e-15.)  A transform is a Stockham sequence of passes of radix 2, 3, 4, 5 or 8
-// through one LDS image per line: a workgroup reads all its butterflies into registers, waits,
-// and writes them back, so one image is enough.  The inverse's last pass and the forward's first
-// have the same radix R (4, 6 or 10): a butterfly's outputs x = j + i X/R of the one are its
-// inputs of the other, so the physical values u, v, w and their products never leave the
-// registers of the thread that owns butterfly j of a pair of lines.
+// Two neighbouring lines share a complex transform, for each of u, v, w and each product, so a line costs 1.5
+// inverse and 3 forward complex transforms of X points.  (Sharing it between u and v of a line, and between uu
+// and vv, leaves the rounding of the larger in the smaller: at 384 x 128 x 257^2 the v and w components of a
+// duct flow's advection were 7.9e-15 and 6.4e-15 off, now 5.3e-15 and 5.4e-15; with rocFFT's transforms of one
+// real line each 5.6e-15 and 5.5e-15.  A value that is not finite spreads to both lines.)  A transform is a
+// Stockham sequence of passes of radix 2, 3, 4, 5 or 8 through one LDS image per line: a workgroup reads all
+// its butterflies into registers, waits, and writes them back, so one image is enough.  The inverse's last
+// pass and the forward's first have the same radix R (4, 6 or 10): a butterfly's outputs x = j + i X/R of the
+// one are its inputs of the other, so the physical values u, v, w and their products never leave the registers
+// of the thread that owns butterfly j of a pair of lines.
 //
 // A workgroup owns T consecutive lines (of the plane's m^2, y fastest): for each mode a run of
 // 16 T bytes, read and written by consecutive lanes.  Lines are padded by one complex value in

@@ -156,7 +156,8 @@ int duct_helm3d_batch_noalloc_dev_(const int *nfields, const duct_devptr_t *rhs,
  * each step (the last one after the final correction) and max|f|, over the
  * refined modes (schemes 5 and 6: not the FP64-solved low Neumann modes).
  * Schemes 5 and 6 without stats are solved in unfolded FP64 at the sizes where
- * that takes less time (planes far below the folded solve's padded size).    */
+ * that takes less time (planes far below the folded solve's padded size, or few
+ * enough for the chip to solve in LDS).                                       */
 int duct_helm3d_mixed_batch_dev_(const int *nfields, const duct_devptr_t *rhs,
                                  const duct_devptr_t *sol, const char *bounds,
                                  const double *alambda, const int *m, const int *nmodes,
