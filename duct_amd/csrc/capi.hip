@@ -148,7 +148,7 @@ struct Lib {
     int fold = 0;                         // 1: Dirichlet groups use the folded passes, 2: Neumann too
     int fuse_quarters = 1;                // folded passes 2 and 3 on LDS-resident quarters where built
     // Tables of the x grids, kept per size until duct_shutdown_: a captured graph and a program that alternates
-    // grids go on using theirs.  At most 48 sizes of the dense transforms (10 MB), 120 of k_xprod_fft (2 MB).
+    // grids go on using theirs.  At most 48 sizes of the dense transforms (13 MB), 86 of k_xprod_fft (1 MB).
     std::map<std::pair<int, int>, XdftTables> xdft;   // dense x-DFTs by (M, X)
     std::map<int, d2v*> xtw;              // roots of unity of k_xprod_fft by X (build_xfft_table)
     d2v* xlane = nullptr;                  // twiddles of the 192-point lane FFTs (build_xlane_table)
