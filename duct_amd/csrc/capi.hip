@@ -2287,6 +2287,8 @@ int duct_advection_dev_(const duct_devptr_t* u, const duct_devptr_t* v, const du
         if (!in[i] || !out[i]) return fail(ERR_ARG, "null device pointer");
         for (int j = 0; j < 3; ++j)
             if (out[i] == in[j]) return fail(ERR_ARG, "adv%d aliases an input velocity", i + 1);
+        for (int j = 0; j < i; ++j)
+            if (out[i] == out[j]) return fail(ERR_ARG, "adv%d and adv%d alias", j + 1, i + 1);
     }
     int st = ensure_init();
     if (st) return st;

@@ -291,7 +291,7 @@ int duct_derivx_dev_(const duct_devptr_t *in, const duct_devptr_t *out, const in
  * src/chebyshev.f90).  Needs duct_setup_ for m and an even mgalx >= 3 nmodes
  * (one fused kernel for mgalx of factors 2, 3 and 5 up to 2048; other grids as dense
  * x-DFTs up to 64 modes and 192 points, through rocFFT past that).  The adv fields must
- * not alias u, v, w.  The reference's slip-velocity, CFL and statistics side
+ * not alias u, v, w or each other.  The reference's slip-velocity, CFL and statistics side
  * outputs of advection3d are not computed.                                  */
 int duct_advection_dev_(const duct_devptr_t *u, const duct_devptr_t *v, const duct_devptr_t *w,
                         const duct_devptr_t *adv1, const duct_devptr_t *adv2, const duct_devptr_t *adv3,
